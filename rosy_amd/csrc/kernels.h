@@ -236,12 +236,14 @@ struct NmEvalLaunch {
     uint32_t L;
     const void* slots;
     uint32_t n_slots;
-    const uint32_t* block_base;  // [slots + 1] first 16x16-texel block of each slot
+    const uint32_t* block_base;  // [slots + 1] first tile of each slot
     const TexGPU* textures;
     const uint8_t* texels;
     const float* srgb_lut;
-    float* partial;  // per block: sum of squared errors over its texels and 7 channels
+    float* partial;  // per tile: sum of squared errors over its texels and 7 channels
+    double* sum;     // per slot
 };
+constexpr uint32_t kNmEvalW = 64, kNmEvalH = 16;  // texels of an evaluation tile
 
 // Decode (or sample the plain maps) at explicit (slot, uv) points.
 struct NmPointLaunch {
@@ -280,10 +282,12 @@ hipError_t launch_blend_fragments(const BlendLaunch& b, const ShadeLaunch& l, hi
 hipError_t launch_blend_resolve(const BlendLaunch& b, const ShadeLaunch& l, hipStream_t s);
 hipError_t launch_nm_init(const NmInitLaunch& l, hipStream_t s);
 hipError_t launch_nm_step(const NmTrainLaunch& l, bool explicit_batch, hipStream_t s);
-hipError_t launch_nm_export(const float* lat, uint4* lat16, uint64_t cells, hipStream_t s);
-hipError_t launch_nm_export_weights(const float* mlp, void* weights, uint32_t fp8, hipStream_t s);
+// the inference parameters: latents as halves, the MLP in its matrix-operand form
+hipError_t launch_nm_export(const float* lat, uint4* lat16, uint64_t cells, const float* mlp, void* weights,
+                            uint32_t fp8, hipStream_t s);
 hipError_t launch_nm_unpack_weights(const void* weights, float* mlp, hipStream_t s);
-hipError_t launch_nm_eval(const NmEvalLaunch& l, uint32_t n_blocks, hipStream_t s);
+// max_tiles: the largest slot's tiles; whether some slot's maps share one extent / differ in size
+hipError_t launch_nm_eval(const NmEvalLaunch& l, uint32_t max_tiles, bool any_same, bool any_other, hipStream_t s);
 hipError_t launch_nm_points(const NmPointLaunch& l, hipStream_t s);
 
 }  // namespace rsy

@@ -86,8 +86,8 @@ __device__ inline void nm_target(const uint8_t* texels, const TexGPU* textures, 
 
 // Inference features of one pixel from the FP16 latent grid of its material (L x L cells of
 // 8 halves = 16 bytes; L a power of two), interpolated in FP32: f[0..7] latent channels,
-// f[8], f[9] positional, f[10] = 1 (carries b1).
-constexpr int kNmFeat = 11;
+// f[8], f[9] positional.
+constexpr int kNmFeat = 10;
 __device__ inline void nm_features(const uint4* grid, uint32_t L, float u, float v, float f[kNmFeat]) {
     const float x = u * float(L) - 0.5f, y = v * float(L) - 0.5f;
     const float fx = floorf(x), fy = floorf(y);
@@ -112,18 +112,37 @@ __device__ inline void nm_features(const uint4* grid, uint32_t L, float u, float
     }
     f[8] = 1.f - fabsf(2.f * ax - 1.f);
     f[9] = 1.f - fabsf(2.f * ay - 1.f);
-    f[10] = 1.f;
 }
 
 // FP32 values as unevaluated sums of two halves: hi = fp16(x), lo = fp16(x - hi) (|error| about
 // 2^-22 |x|).  Products with FP16 weights are exact in the MFMA's FP32 accumulation, so feeding hi
 // and lo as two B operands gives W x to FP32-level accuracy for the FP16 weights.
-__device__ inline void nm_split8(const float (&x)[8], h8& hi, h8& lo) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        hi[k] = _Float16(x[k]);
-        lo[k] = _Float16(x[k] - float(hi[k]));
-    }
+// In pairs: one v_cvt_pk_f16_f32 for two values, and each remainder x - float(half), rounded to a half, as one
+// v_fma_mix{lo,hi}_f16.  `minus1` is -1 in a register the compiler cannot see through: it would widen
+// each half, subtract and convert instead (3.5 instructions a value against 1.5).
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+__device__ inline float nm_opaque(float m) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+s"(m));
+#endif
+    return m;
+}
+__device__ inline void nm_split2(float x0, float x1, float minus1, uint32_t& hi, uint32_t& lo) {
+    hi = __builtin_bit_cast(uint32_t, h2{_Float16(x0), _Float16(x1)});
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(hi));  // the remainders read this packed word (not conversions of their own)
+#endif
+    const h2 h = __builtin_bit_cast(h2, hi);
+    lo = __builtin_bit_cast(uint32_t, h2{_Float16(fmaf(float(h[0]), minus1, x0)), _Float16(fmaf(float(h[1]), minus1, x1))});
+}
+__device__ inline void nm_split8(const float (&x)[8], float minus1, h8& hi, h8& lo) {
+    uint4 h, l;
+    nm_split2(x[0], x[1], minus1, h.x, l.x);
+    nm_split2(x[2], x[3], minus1, h.y, l.y);
+    nm_split2(x[4], x[5], minus1, h.z, l.z);
+    nm_split2(x[6], x[7], minus1, h.w, l.w);
+    hi = __builtin_bit_cast(h8, h);
+    lo = __builtin_bit_cast(h8, l);
 }
 
 // Eight E4M3 codes widened to FP16: sign to bit 15, exponent and mantissa to bits 13..7.  Exact for
@@ -138,34 +157,37 @@ __device__ inline h8 nm_widen_e4m3(uint2 q) {
     return r;
 }
 
-__device__ inline h8 nm_swap_halves(h8 v) {  // value of lane l ^ 32
-    const int addr = int((nm_lane() ^ 32u) << 2);
-    uint4 b = __builtin_bit_cast(uint4, v);
-    b.x = uint32_t(__builtin_amdgcn_ds_bpermute(addr, int(b.x)));
-    b.y = uint32_t(__builtin_amdgcn_ds_bpermute(addr, int(b.y)));
-    b.z = uint32_t(__builtin_amdgcn_ds_bpermute(addr, int(b.z)));
-    b.w = uint32_t(__builtin_amdgcn_ds_bpermute(addr, int(b.w)));
-    return __builtin_bit_cast(h8, b);
+// Exchanges lanes 32..63 of `a` with lanes 0..31 of `b` (v_permlane32_swap_b32: one VALU move per word,
+// where two LDS permutes and their selects took about ten instructions and a round trip).
+__device__ inline void nm_swap32(uint32_t& a, uint32_t& b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+#endif
 }
-
-__device__ inline float nm_swap_f(float v) {
-    const int addr = int((nm_lane() ^ 32u) << 2);
-    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(v)));
+__device__ inline void nm_swap32(h8& a, h8& b) {
+    uint4 x = __builtin_bit_cast(uint4, a), y = __builtin_bit_cast(uint4, b);
+    nm_swap32(x.x, y.x);
+    nm_swap32(x.y, y.y);
+    nm_swap32(x.z, y.z);
+    nm_swap32(x.w, y.w);
+    a = __builtin_bit_cast(h8, x);
+    b = __builtin_bit_cast(h8, y);
 }
 
 // MLP of the 64 pixels of a wave, one pixel per lane (features f from nm_features); every lane of
 // the wave must call it with the wave fully active.  Returns this lane's 7 clamped outputs.
 //
 // Pixel tile t (t = 0, 1) is lanes 32t .. 32t + 31.  The B operand of layer 1 for tile t, lane l is
-// features 8 (l / 32) .. +7 of pixel 32t + l % 32: a lane holds its own pixel's features and swaps
-// the other half with lane l ^ 32.  The layer-1 accumulator of lane l holds hidden rows
+// features 8 (l / 32) .. +7 of pixel 32t + l % 32: exchanging the upper lanes of the first feature
+// half with the lower lanes of the second gives both tiles' operands.  The layer-1 accumulator of lane l holds hidden rows
 // 8 (r / 4) + 4 (l / 32) + r % 4 (r = 0..15) of pixel l % 32; after ReLU, entries 8s .. 8s + 7 are
 // layer 2's B operand for K-step s.  Output rows 0..7 land in accumulator entries 0..3: rows 0-3 in
 // lanes 0-31 and rows 4-7 in lanes 32-63 of the same column.  Every B operand goes in as an FP16
 // hi / lo pair (nm_split8).
 __device__ inline void nm_mlp_wave(const NmWeights* __restrict__ W, const float f[kNmFeat], float out[kNmOut]) {
     const uint32_t lane = nm_lane();
-    const bool hi = lane >= 32u;
     h8 a1, a2[2];
     if (W->fp8) {  // uniform: one weight form per decoder
         a1 = nm_widen_e4m3(W->q1[lane]);
@@ -178,52 +200,49 @@ __device__ inline void nm_mlp_wave(const NmWeights* __restrict__ W, const float 
     }
     // feature halves: 0..7 the latent channels; 8..15 the positional pair, the constant 1, zeros
     const float g0[8] = {f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
-    const float g1[8] = {f[8], f[9], f[10], 0.f, 0.f, 0.f, 0.f, 0.f};
-    h8 q0h, q0l, q1h, q1l;
-    nm_split8(g0, q0h, q0l);
-    nm_split8(g1, q1h, q1l);
-    // tile t wants half (l / 32) of pixel 32t + l % 32: the lane's own features for t == l / 32,
-    // otherwise those of lane l ^ 32 (which sends the half this lane needs)
-    const h8 own_h = hi ? q1h : q0h, own_l = hi ? q1l : q0l;
-    const h8 far_h = nm_swap_halves(hi ? q0h : q1h), far_l = nm_swap_halves(hi ? q0l : q1l);
-    const float s1 = W->scale[0], s2 = W->scale[1];
-    float res[2][4];
+    const float minus1 = nm_opaque(-1.0f);
+    // ReLU as the median of x, 0 and infinity: one instruction (NaN gives 0 as fmaxf does), where fmaxf
+    // on a matrix result takes two (the first quiets a signalling NaN)
+    const float inf = nm_opaque(__builtin_inff());
+    h8 q0h, q0l;
+    nm_split8(g0, minus1, q0h, q0l);
+    uint4 ph = make_uint4(0u, 0x3c00u, 0u, 0u), pl = make_uint4(0u, 0u, 0u, 0u);  // 0x3c00: 1 as a half
+    nm_split2(f[8], f[9], minus1, ph.x, pl.x);
+    h8 q1h = __builtin_bit_cast(h8, ph), q1l = __builtin_bit_cast(h8, pl);
+    nm_swap32(q0h, q1h);  // q0: tile 0's operand (lower lanes the first half, upper lanes the second), q1: tile 1's
+    nm_swap32(q0l, q1l);
+    // both layers' scales are applied to the outputs: relu(s1 x) = s1 relu(x) for s1 > 0
+    const float s12 = W->scale[0] * W->scale[1];
+    uint32_t res[2][4];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const bool own = (t == 1) == hi;
         f32x16 acc = {};
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, own ? own_h : far_h, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, own ? own_l : far_l, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, t == 0 ? q0h : q1h, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, t == 0 ? q0l : q1l, acc, 0, 0, 0);
         f32x16 acc2 = {};
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             float h[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) h[j] = fmaxf(acc[8 * s + j] * s1, 0.f);
+            for (int j = 0; j < 8; ++j) h[j] = __builtin_amdgcn_fmed3f(acc[8 * s + j], 0.f, inf);
             h8 hh, hl;
-            nm_split8(h, hh, hl);
+            nm_split8(h, minus1, hh, hl);
             acc2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[s], hh, acc2, 0, 0, 0);
             acc2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[s], hl, acc2, 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) res[t][r] = acc2[r];
+        for (int r = 0; r < 4; ++r) res[t][r] = __float_as_uint(acc2[r]);
     }
-    // own pixel = tile (hi ? 1 : 0): rows 4*hi .. +3 here, the other four rows in lane l ^ 32
-    float own_rows[4], far_rows[4];
+    // rows 0..3 of tile t are in its lower lanes, rows 4..7 in its upper ones: the same exchange
+    // leaves every lane its own pixel's rows 0..3 in res[0] and 4..7 in res[1]
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        own_rows[r] = hi ? res[1][r] : res[0][r];
-        far_rows[r] = nm_swap_f(hi ? res[0][r] : res[1][r]);
+        nm_swap32(res[0][r], res[1][r]);
+        out[r] = __uint_as_float(res[0][r]);
+        if (r < 3) out[4 + r] = __uint_as_float(res[1][r]);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float lo4 = hi ? far_rows[r] : own_rows[r];  // rows 0..3
-        const float hi4 = hi ? own_rows[r] : far_rows[r];  // rows 4..7
-        out[r] = lo4;
-        if (r < 3) out[4 + r] = hi4;
-    }
-#pragma unroll
-    for (int c = 0; c < kNmOut; ++c) out[c] = fminf(1.f, fmaxf(0.f, out[c] * s2 + W->b2[c]));
+    for (int c = 0; c < kNmOut; ++c) out[c] = __builtin_amdgcn_fmed3f(fmaf(out[c], s12, W->b2[c]), 0.f, 1.f);
 }
 
 }  // namespace rsy

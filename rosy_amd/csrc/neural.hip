@@ -304,11 +304,20 @@ __global__ __launch_bounds__(256) void k_nm_init(NmInitLaunch I) {
     }
 }
 
-__global__ __launch_bounds__(256) void k_nm_export(const float* lat, uint4* lat16, uint64_t cells) {
-    for (uint64_t cell = uint64_t(blockIdx.x) * 256 + threadIdx.x; cell < cells; cell += uint64_t(gridDim.x) * 256) {
+// FP32 latents to halves; the last block's first wave writes the MLP's operand form instead (a launch
+// of its own took 8 us beside the latents' 17).
+__device__ void export_weights(const float* p, NmWeights* W, uint32_t fp8);
+
+__global__ __launch_bounds__(256) void k_nm_export(const float* lat, uint4* lat16, uint64_t cells, const float* mlp,
+                                                   NmWeights* W, uint32_t fp8) {
+    if (blockIdx.x + 1 == gridDim.x) {
+        if (threadIdx.x < 64) export_weights(mlp, W, fp8);
+        return;
+    }
+    const uint32_t blocks = gridDim.x - 1;
+    for (uint64_t cell = uint64_t(blockIdx.x) * 256 + threadIdx.x; cell < cells; cell += uint64_t(blocks) * 256) {
         const float4 a = reinterpret_cast<const float4*>(lat)[2 * cell];
         const float4 b = reinterpret_cast<const float4*>(lat)[2 * cell + 1];
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
         const h2 p0 = h2{_Float16(a.x), _Float16(a.y)}, p1 = h2{_Float16(a.z), _Float16(a.w)};
         const h2 p2 = h2{_Float16(b.x), _Float16(b.y)}, p3 = h2{_Float16(b.z), _Float16(b.w)};
         lat16[cell] = make_uint4(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1),
@@ -316,31 +325,130 @@ __global__ __launch_bounds__(256) void k_nm_export(const float* lat, uint4* lat1
     }
 }
 
-// One block = a 16 x 16 texel tile of one slot's albedo map; all 256 lanes run the MLP.
+// Two neighbouring cells of a latent grid interpolated.
+__device__ inline void nm_row(uint4 a, uint4 b, float t, float (&out)[kNmCh]) {
+    const uint32_t p[4] = {a.x, a.y, a.z, a.w}, q[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const h2 x = __builtin_bit_cast(h2, p[k]), y = __builtin_bit_cast(h2, q[k]);
+        out[2 * k] = (1.f - t) * float(x[0]) + t * float(y[0]);
+        out[2 * k + 1] = (1.f - t) * float(x[1]) + t * float(y[1]);
+    }
+}
+
+// Squared error of the decoder over every texel centre of one slot's albedo map, a block per tile of
+// kNmEvalW x kNmEvalH texels: lane = column, a wave walks kNmEvalH / 4 rows.
+//
+// kTexel: the slot's three maps share one extent, so that the plain sampler at a texel centre is the
+// texel itself (bilinear weights 1, 0, 0, 0): three loads and seven table reads, against twelve loads
+// with addressing and format branches.  Slots whose maps differ in size sample bilinearly
+// (kTexel = false); each launch passes over the other kind's slots.
+//
+// Bound by VALU issue: 64 texels take about 230 instructions of 4 cycles (half splits, clamps, error) next to 12
+// matrix instructions of 32; texels and latents are 12 bytes a texel.  The rows of a wave share the
+// weights, the column's addresses and most cell rows.  32 materials of 1024^2 texels with 256^2 latents: 850 us
+// with 256-texel blocks, four cells and twelve texels per texel, 350 us this way (49 us of
+// memory time; 16 rows a wave: 344 us, at 3 waves a SIMD instead of 4).
+template <bool kTexel>
 __global__ __launch_bounds__(256) void k_nm_eval(NmEvalLaunch E) {
     __shared__ float red_s[4];
-    uint32_t slot = 0;
-    while (slot + 1 < E.n_slots && E.block_base[slot + 1] <= blockIdx.x) ++slot;
-    const NmSlot S = static_cast<const NmSlot*>(E.slots)[slot];
-    const TexGPU ta = E.textures[S.albedo];
-    const uint32_t tiles_x = (ta.width + 15) / 16;
-    const uint32_t tb = blockIdx.x - E.block_base[slot];
-    const uint32_t tx = (tb % tiles_x) * 16 + (threadIdx.x & 15), ty = (tb / tiles_x) * 16 + (threadIdx.x >> 4);
-    const bool valid = tx < ta.width && ty < ta.height;
-    const float u = (float(tx) + 0.5f) / float(ta.width), v = (float(ty) + 0.5f) / float(ta.height);
-    float f[kNmFeat];
-    nm_features(E.lat16 + size_t(slot) * E.L * E.L, E.L, u, v, f);
-    float dec[kNmOut];
-    nm_mlp_wave(static_cast<const NmWeights*>(E.weights), f, dec);
-    float err = 0.f;
-    if (valid) {
-        float tgt[kNmOut];
-        nm_target(E.texels, E.textures, S, u, v, E.srgb_lut, tgt);
+    __shared__ float lut[2][256];  // stored byte -> value: UNORM, sRGB
+    lut[0][threadIdx.x] = float(threadIdx.x) * (1.0f / 255.0f);
+    lut[1][threadIdx.x] = E.srgb_lut[threadIdx.x];
+    __syncthreads();
+    for (uint32_t slot = blockIdx.y; slot < E.n_slots; slot += gridDim.y) {
+        const NmSlot S = static_cast<const NmSlot*>(E.slots)[slot];
+        const TexGPU ta = E.textures[S.albedo], tn = E.textures[S.normal], tm = E.textures[S.mr];
+        const bool same = tn.width == ta.width && tn.height == ta.height && tm.width == ta.width && tm.height == ta.height;
+        const uint32_t tiles_x = (ta.width + kNmEvalW - 1) / kNmEvalW, tiles_y = (ta.height + kNmEvalH - 1) / kNmEvalH;
+        if (same != kTexel || blockIdx.x >= tiles_x * tiles_y) continue;  // uniform
+        const uint32_t x = (blockIdx.x % tiles_x) * kNmEvalW + (threadIdx.x & 63u);
+        const uint32_t y0 = (blockIdx.x / tiles_x) * kNmEvalH +
+                            uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))) * (kNmEvalH / 4);
+        const uint32_t xc = min(x, ta.width - 1);
+        const float u = (float(xc) + 0.5f) / float(ta.width);
+        const uint32_t* albedo = reinterpret_cast<const uint32_t*>(E.texels + ta.offset) + xc;
+        const uint16_t* normal = reinterpret_cast<const uint16_t*>(E.texels + tn.offset) + xc;
+        const uint16_t* mr = reinterpret_cast<const uint16_t*>(E.texels + tm.offset) + xc;
+        const float *la = lut[ta.srgb ? 1 : 0], *ln = lut[tn.srgb ? 1 : 0], *lm = lut[tm.srgb ? 1 : 0];
+        const uint4* grid = E.lat16 + size_t(slot) * E.L * E.L;
+        // the column's two cell columns and weight; the two cell rows around a texel row, interpolated
+        // along x and kept while the next texel row lies between the same ones (rows are uniform over the wave)
+        const float gx = u * float(E.L) - 0.5f, fx = floorf(gx), ax = gx - fx;
+        const uint32_t mask = E.L - 1, cx0 = uint32_t(int(fx)) & mask, cx1 = (cx0 + 1) & mask;
+        float lower[kNmCh], slope[kNmCh], upper[kNmCh];  // row cy, row cy + 1 less row cy, row cy + 1
+        uint32_t at = 0xffffffffu;                       // the row in `lower` (none yet)
+        float err = 0.f;
+        for (uint32_t j = 0; j < kNmEvalH / 4; ++j) {
+            const uint32_t yc = min(y0 + j, ta.height - 1);
+            const float v = (float(yc) + 0.5f) / float(ta.height);
+            const size_t row = size_t(yc) * ta.width;
+            uint32_t pa = 0, pn = 0, pm = 0;
+            if constexpr (kTexel) {
+                pa = albedo[row];
+                pn = normal[row];
+                pm = mr[row];
+            }
+            const float gy = v * float(E.L) - 0.5f, fy = floorf(gy), ay = gy - fy;
+            const uint32_t cy = uint32_t(int(fy)) & mask;
+            if (cy != at) {
+                if (at != 0xffffffffu && cy == ((at + 1) & mask)) {
 #pragma unroll
-        for (int c = 0; c < kNmOut; ++c) err += (dec[c] - tgt[c]) * (dec[c] - tgt[c]);
+                    for (int c = 0; c < kNmCh; ++c) lower[c] = upper[c];
+                } else {
+                    nm_row(grid[cy * E.L + cx0], grid[cy * E.L + cx1], ax, lower);
+                }
+                const uint32_t cy1 = (cy + 1) & mask;
+                nm_row(grid[cy1 * E.L + cx0], grid[cy1 * E.L + cx1], ax, upper);
+#pragma unroll
+                for (int c = 0; c < kNmCh; ++c) slope[c] = upper[c] - lower[c];
+                at = cy;
+            }
+            float f[kNmFeat];
+#pragma unroll
+            for (int c = 0; c < kNmCh; ++c) f[c] = fmaf(ay, slope[c], lower[c]);
+            f[8] = 1.f - fabsf(2.f * ax - 1.f);
+            f[9] = 1.f - fabsf(2.f * ay - 1.f);
+            float dec[kNmOut];
+            nm_mlp_wave(static_cast<const NmWeights*>(E.weights), f, dec);
+            float tgt[kNmOut];
+            if constexpr (kTexel) {
+                tgt[0] = la[pa & 0xffu];
+                tgt[1] = la[(pa >> 8) & 0xffu];
+                tgt[2] = la[(pa >> 16) & 0xffu];
+                tgt[3] = ln[pn & 0xffu];
+                tgt[4] = ln[pn >> 8];
+                tgt[5] = lm[pm & 0xffu];
+                tgt[6] = lm[pm >> 8];
+            } else {
+                nm_target(E.texels, E.textures, S, u, v, lut[1], tgt);
+            }
+            float e = 0.f;
+#pragma unroll
+            for (int c = 0; c < kNmOut; ++c) e += (dec[c] - tgt[c]) * (dec[c] - tgt[c]);
+            if (x < ta.width && y0 + j < ta.height) err += e;
+        }
+        const float s = block_sum(err, red_s);
+        if (threadIdx.x == 0) E.partial[E.block_base[slot] + blockIdx.x] = s;
+        __syncthreads();  // red_s is written again for the next slot
     }
-    const float s = block_sum(err, red_s);
-    if (threadIdx.x == 0) E.partial[blockIdx.x] = s;
+}
+
+// One block per slot: its tiles' sums in FP64, in a fixed order (the host reads one value a slot
+// instead of one a tile).
+__global__ __launch_bounds__(256) void k_nm_eval_sum(NmEvalLaunch E) {
+    __shared__ double red[256];
+    for (uint32_t slot = blockIdx.x; slot < E.n_slots; slot += gridDim.x) {
+        double s = 0.0;
+        for (uint32_t b = E.block_base[slot] + threadIdx.x; b < E.block_base[slot + 1]; b += 256) s += double(E.partial[b]);
+        red[threadIdx.x] = s;
+        for (uint32_t o = 128; o > 0; o >>= 1) {
+            __syncthreads();
+            if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+        }
+        if (threadIdx.x == 0) E.sum[slot] = red[0];
+        __syncthreads();
+    }
 }
 
 __global__ __launch_bounds__(256) void k_nm_points(NmPointLaunch P) {
@@ -370,7 +478,7 @@ __device__ inline float layer_weight(const float* p, int layer, uint32_t i, uint
     return i < uint32_t(kNmOut) ? p[kNmW2 + i * kNmHidden + k] : 0.f;
 }
 
-__global__ __launch_bounds__(64) void k_nm_export_weights(const float* p, NmWeights* W, uint32_t fp8) {
+__device__ void export_weights(const float* p, NmWeights* W, uint32_t fp8) {
     const uint32_t l = threadIdx.x, i = l % 32, hb = l / 32;
     float scale[2] = {1.f, 1.f};
     if (fp8) {
@@ -430,11 +538,6 @@ __global__ __launch_bounds__(64) void k_nm_unpack_weights(const NmWeights* W, fl
 
 }  // namespace
 
-hipError_t launch_nm_export_weights(const float* mlp, void* weights, uint32_t fp8, hipStream_t s) {
-    hipLaunchKernelGGL(k_nm_export_weights, dim3(1), dim3(64), 0, s, mlp, static_cast<NmWeights*>(weights), fp8);
-    return hipGetLastError();
-}
-
 hipError_t launch_nm_unpack_weights(const void* weights, float* mlp, hipStream_t s) {
     hipLaunchKernelGGL(k_nm_unpack_weights, dim3(1), dim3(64), 0, s, static_cast<const NmWeights*>(weights), mlp);
     return hipGetLastError();
@@ -462,16 +565,20 @@ hipError_t launch_nm_step(const NmTrainLaunch& l, bool explicit_batch, hipStream
     return hipGetLastError();
 }
 
-hipError_t launch_nm_export(const float* lat, uint4* lat16, uint64_t cells, hipStream_t s) {
+hipError_t launch_nm_export(const float* lat, uint4* lat16, uint64_t cells, const float* mlp, void* weights,
+                            uint32_t fp8, hipStream_t s) {
     const uint32_t blocks = uint32_t(std::min<uint64_t>((cells + 255) / 256, 65536));
-    if (blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_nm_export, dim3(blocks), dim3(256), 0, s, lat, lat16, cells);
+    hipLaunchKernelGGL(k_nm_export, dim3(blocks + 1), dim3(256), 0, s, lat, lat16, cells, mlp,
+                       static_cast<NmWeights*>(weights), fp8);
     return hipGetLastError();
 }
 
-hipError_t launch_nm_eval(const NmEvalLaunch& l, uint32_t n_blocks, hipStream_t s) {
-    if (n_blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_nm_eval, dim3(n_blocks), dim3(256), 0, s, l);
+hipError_t launch_nm_eval(const NmEvalLaunch& l, uint32_t max_tiles, bool any_same, bool any_other, hipStream_t s) {
+    if (l.n_slots == 0 || max_tiles == 0) return hipSuccess;
+    const dim3 grid(max_tiles, min(l.n_slots, 65535u));
+    if (any_same) hipLaunchKernelGGL(k_nm_eval<true>, grid, dim3(256), 0, s, l);
+    if (any_other) hipLaunchKernelGGL(k_nm_eval<false>, grid, dim3(256), 0, s, l);
+    hipLaunchKernelGGL(k_nm_eval_sum, dim3(min(l.n_slots, 65535u)), dim3(256), 0, s, l);
     return hipGetLastError();
 }
 

@@ -25,9 +25,11 @@ struct NeuralState {
     std::vector<uint32_t> slot_of;  // per material: slot or 0xFFFFFFFF
     std::vector<uint32_t> active;   // per material
     std::vector<float> psnr;        // per material (NaN: not eligible / not evaluated)
-    std::vector<uint32_t> block_base;  // evaluation blocks per slot (prefix, n_slots + 1)
+    std::vector<uint32_t> block_base;  // evaluation tiles per slot (prefix, n_slots + 1)
+    uint32_t max_tiles = 0;            // of the largest slot
+    bool any_same = false, any_other = false;  // some slot's maps share one extent / differ in size
     DevBuf slots_d, slot_of_d, active_d, block_base_d;
-    DevBuf lat, lat_m, lat_v, mlp, mlp_m, mlp_v, partial, step_d, loss_d, lat16, weights_d, eval_partial;
+    DevBuf lat, lat_m, lat_v, mlp, mlp_m, mlp_v, partial, step_d, loss_d, lat16, weights_d, eval_partial, eval_sum;
     DevBuf tmp[5];
     uint32_t n_wg = 0, spw = 0;
     uint32_t steps = 0;
@@ -222,11 +224,16 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     const uint64_t n_regions = std::max<uint64_t>(1, uint64_t(ns) * rpm);
     n->n_wg = uint32_t(std::min<uint64_t>(cfg->batch / 256, n_regions));
     n->spw = (cfg->batch + n->n_wg - 1) / n->n_wg;
-    // evaluation blocks: 16 x 16 texel tiles of each slot's albedo map
+    // evaluation tiles of each slot's albedo map
     n->block_base.assign(ns + 1, 0);
     for (uint32_t i = 0; i < ns; ++i) {
-        const TexGPU& t = c->h_tex_table[n->slots[i].albedo];
-        n->block_base[i + 1] = n->block_base[i] + ((t.width + 15) / 16) * ((t.height + 15) / 16);
+        const NmSlot& sl = n->slots[i];
+        const TexGPU &t = c->h_tex_table[sl.albedo], &tn = c->h_tex_table[sl.normal], &tm = c->h_tex_table[sl.mr];
+        const uint32_t tiles = ((t.width + kNmEvalW - 1) / kNmEvalW) * ((t.height + kNmEvalH - 1) / kNmEvalH);
+        n->block_base[i + 1] = n->block_base[i] + tiles;
+        n->max_tiles = std::max(n->max_tiles, tiles);
+        const bool same = tn.width == t.width && tn.height == t.height && tm.width == t.width && tm.height == t.height;
+        (same ? n->any_same : n->any_other) = true;
     }
     hipStream_t s = c->stream;
     HIP_TRY(c, hipEventCreate(&n->ev0), "event");
@@ -247,7 +254,8 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
             "allocate decoder");
     HIP_TRY(c, n->step_d.ensure(4), "allocate decoder");
     HIP_TRY(c, n->weights_d.ensure(kNmWeightsBytes), "allocate decoder");
-    HIP_TRY(c, n->eval_partial.ensure(std::max<uint32_t>(1, n->block_base[ns]) * 4), "allocate decoder");
+    HIP_TRY(c, n->eval_partial.ensure(size_t(std::max<uint32_t>(1, n->block_base[ns])) * 4), "allocate decoder");
+    HIP_TRY(c, n->eval_sum.ensure(std::max<size_t>(1, ns) * 8), "allocate decoder");
     if (ns) HIP_TRY(c, hipMemcpy(n->slots_d.p, n->slots.data(), ns * sizeof(NmSlot), hipMemcpyHostToDevice), "upload");
     if (nm) {
         HIP_TRY(c, hipMemcpy(n->slot_of_d.p, n->slot_of.data(), nm * 4, hipMemcpyHostToDevice), "upload");
@@ -332,9 +340,9 @@ rsy_result rsy_neural_evaluate(rsy_ctx* c, float* psnr, uint32_t n_materials) {
     HIP_TRY(c, hipStreamSynchronize(s), "synchronize");
     const uint32_t ns = uint32_t(n->slots.size());
     HIP_TRY(c, hipEventRecord(n->ev0, s), "event");
-    HIP_TRY(c, launch_nm_export(n->lat.as<float>(), n->lat16.as<uint4>(), uint64_t(ns) * n->L * n->L, s), "export latents");
-    HIP_TRY(c, launch_nm_export_weights(n->mlp.as<float>(), n->weights_d.p, n->cfg.weights == RSY_NEURAL_WEIGHTS_FP8 ? 1u : 0u, s),
-            "export weights");
+    HIP_TRY(c, launch_nm_export(n->lat.as<float>(), n->lat16.as<uint4>(), uint64_t(ns) * n->L * n->L, n->mlp.as<float>(),
+                                n->weights_d.p, n->cfg.weights == RSY_NEURAL_WEIGHTS_FP8 ? 1u : 0u, s),
+            "export inference parameters");
     NmEvalLaunch E{};
     E.lat16 = n->lat16.as<uint4>();
     E.weights = n->weights_d.p;
@@ -346,18 +354,16 @@ rsy_result rsy_neural_evaluate(rsy_ctx* c, float* psnr, uint32_t n_materials) {
     E.texels = c->texels.as<uint8_t>();
     E.srgb_lut = c->srgb_lut.as<float>();
     E.partial = n->eval_partial.as<float>();
-    const uint32_t blocks = n->block_base[ns];
-    HIP_TRY(c, launch_nm_eval(E, blocks, s), "evaluate decoder");
+    E.sum = n->eval_sum.as<double>();
+    HIP_TRY(c, launch_nm_eval(E, n->max_tiles, n->any_same, n->any_other, s), "evaluate decoder");
     HIP_TRY(c, hipEventRecord(n->ev1, s), "event");
-    std::vector<float> part(blocks);
-    if (blocks) HIP_TRY(c, hipMemcpyAsync(part.data(), n->eval_partial.p, size_t(blocks) * 4, hipMemcpyDeviceToHost, s), "read");
+    std::vector<double> sums(ns);
+    if (ns) HIP_TRY(c, hipMemcpyAsync(sums.data(), n->eval_sum.p, size_t(ns) * 8, hipMemcpyDeviceToHost, s), "read");
     HIP_TRY(c, hipStreamSynchronize(s), "synchronize");
     HIP_TRY(c, hipEventElapsedTime(&n->eval_ms, n->ev0, n->ev1), "event");
     for (uint32_t i = 0; i < ns; ++i) {
-        double sum = 0.0;
-        for (uint32_t b = n->block_base[i]; b < n->block_base[i + 1]; ++b) sum += part[b];
         const TexGPU& t = c->h_tex_table[n->slots[i].albedo];
-        const double mse = sum / (double(t.width) * t.height * kNmOut);
+        const double mse = sums[i] / (double(t.width) * t.height * kNmOut);
         const double p = mse > 0.0 ? 10.0 * std::log10(1.0 / mse) : INFINITY;
         const uint32_t m = n->slots[i].material;
         n->psnr[m] = float(p);
