@@ -193,13 +193,14 @@ struct NmTrainLaunch {
     float* mlp;      // [584] FP32 MLP parameters (W1, b1, W2, b2)
     float* mlp_m;
     float* mlp_v;
+    float* tables;   // [19][64] the MLP in the step's operand form
     float* partial;  // [n_wg][584]: per-workgroup MLP gradient sums, loss sum at index 583
-    uint32_t* step;  // device step counter: completed Adam steps
+    uint32_t* step;  // device step counter: Adam steps completed before the batch of launches
+    uint32_t step_ahead;  // this launch's step in its batch
     float* loss_out; // loss per step, index step - loss_base (nullable)
     uint32_t loss_base, loss_cap;
-    const void* slots;  // NmSlot
+    const TexGPU* maps;  // [slots][3]: each slot's albedo, normal and metallic-roughness records
     uint32_t n_slots;
-    const TexGPU* textures;
     const uint8_t* texels;
     const float* srgb_lut;
     uint32_t L, log2L;
@@ -281,7 +282,11 @@ hipError_t launch_shade(const ShadeLaunch& l, hipStream_t s);
 hipError_t launch_blend_fragments(const BlendLaunch& b, const ShadeLaunch& l, hipStream_t s);
 hipError_t launch_blend_resolve(const BlendLaunch& b, const ShadeLaunch& l, hipStream_t s);
 hipError_t launch_nm_init(const NmInitLaunch& l, hipStream_t s);
-hipError_t launch_nm_step(const NmTrainLaunch& l, bool explicit_batch, hipStream_t s);
+// the step's weight tables from the MLP (before the first step); `steps` Adam steps (they keep the tables
+// up to date); the exact gradient of the explicit batch
+hipError_t launch_nm_tables(const NmTrainLaunch& l, hipStream_t s);
+hipError_t launch_nm_steps(NmTrainLaunch l, uint32_t steps, hipStream_t s);
+hipError_t launch_nm_gradient(const NmTrainLaunch& l, hipStream_t s);
 // the inference parameters: latents as halves, the MLP in its matrix-operand form
 hipError_t launch_nm_export(const float* lat, uint4* lat16, uint64_t cells, const float* mlp, void* weights,
                             uint32_t fp8, hipStream_t s);

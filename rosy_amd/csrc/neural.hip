@@ -5,18 +5,19 @@
 // sampler's values there (mean squared error over the 7 channels), then applies one Adam update
 // (lr with an optional cosine decay, beta1, beta2, eps) to the latents it touched and to the shared MLP.  Samples are drawn per
 // workgroup inside a region of 2^log2R x 2^log2R latent cells of one material, positioned so that
-// every bilinear footprint stays inside the region: the region's latents and their gradients live
-// in LDS (gradients accumulate with LDS atomics, never with global ones), and the workgroup applies
+// every bilinear footprint stays inside the region: the region's latent gradients live
+// in LDS (they accumulate with LDS atomics, never with global ones), and the workgroup applies
 // Adam to its region itself.  The regions of one step are distinct cells of one partition of every
 // grid (the partition shifts by a random offset each step), so no two workgroups touch the same
 // latent.  The MLP gradient is reduced per workgroup from per-sample records in LDS and summed over
-// workgroups in a fixed order by one wave per parameter, which also applies Adam to it; a last
-// one-thread kernel advances the device-side step counter (so a captured graph of steps replays as
-// consecutive steps).
+// workgroups in a fixed order by a second kernel, which also applies Adam to it; after a batch of
+// steps a one-thread kernel advances the device-side step counter (each launch of the batch knows how
+// many steps it is ahead of it, so a captured graph of steps replays as consecutive steps).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
+#include "bin_raster.h"
 #include "frame_types.h"
 #include "kernels.h"
 #include "neural.h"
@@ -25,8 +26,17 @@ namespace rsy {
 namespace {
 
 constexpr int kMaxR = 32;   // largest region side (explicit mode: the whole grid)
-constexpr int kRec = 81;    // per-sample record: features 10, hidden 32, dL/dout 7, dL/dhidden 32
-constexpr int kRecIn = 0, kRecH = 10, kRecDo = 42, kRecDh = 49;
+// Per-sample record in LDS for the MLP gradient products, in groups of four words: dL/dhidden 32,
+// features 10 and the constant 1 (its products are the bias gradients), dL/dout 7, hidden 32,
+// dL/dlatent 8; the sample's two bilinear weights sit in the feature and output groups' spare words.
+constexpr int kRec = 92, kRecDh = 0, kRecIn = 32, kRecAx = 43, kRecDo = 44, kRecAy = 51, kRecH = 52, kRecDl = 84;
+// The products as 4 x 4 blocks, 16 a wave: dL/dW1 and dL/db1 (8 hidden groups by 3 feature groups),
+// dL/dW2 (8 hidden groups by 2 output groups), dL/db2 (the constant's group by 2 output groups).
+constexpr uint32_t kGradBlocks1 = 24, kGradBlocks2 = 16, kGradBlocks = kGradBlocks1 + kGradBlocks2 + 2;
+constexpr uint32_t kGradWaves = (kGradBlocks + 15) / 16;
+static_assert(kGradWaves <= 4, "the sample waves");
+constexpr uint32_t kStepThreads = 512;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ inline uint64_t mix64(uint64_t z) {  // SplitMix64 finaliser
     z += 0x9E3779B97F4A7C15ull;
@@ -36,6 +46,19 @@ __device__ inline uint64_t mix64(uint64_t z) {  // SplitMix64 finaliser
 }
 
 __device__ inline float unit24(uint32_t x) { return float(x >> 8) * (1.0f / 16777216.0f); }  // [0, 1)
+
+__device__ inline float mul_rn(float a, float b) {  // rounded by itself: not fused into a later sum
+#pragma clang fp contract(off)
+    return a * b;
+}
+
+// One Adam step of a parameter x with moments m, v; `rate` is the learning rate, bc1 and bc2 the moments' corrections.
+__device__ inline void adam_step(float& x, float& m, float& v, float g, const NmTrainLaunch& T, float rate, float bc1,
+                                 float bc2) {
+    m = fmaf(1.f - T.beta1, g, mul_rn(T.beta1, m));
+    v = fmaf(g, mul_rn(1.f - T.beta2, g), mul_rn(T.beta2, v));
+    x = x - rate * (m / bc1) / (sqrtf(v / bc2) + T.eps);
+}
 
 // Learning-rate factor of step `step`: 0.5 (1 + cos(pi step / decay)) until `decay`, then 0.
 __device__ inline float lr_factor(uint32_t step, uint32_t decay) {
@@ -55,26 +78,185 @@ __device__ inline float block_sum(float v, float* red) {
     return s;
 }
 
-template <bool kExplicit>
-__global__ __launch_bounds__(256) void k_nm_step(NmTrainLaunch T) {
-    __shared__ float lat_s[kMaxR * kMaxR * kNmCh];
-    __shared__ float grad_s[kMaxR * kMaxR * kNmCh];
-    __shared__ float w_s[kNmParamsPad];
-    __shared__ float rec_s[256 * kRec];
-    __shared__ float red_s[4];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t step = kExplicit ? 0u : *T.step;
-    const uint32_t L = T.L, Lm = L - 1;
-    const NmSlot* slots = static_cast<const NmSlot*>(T.slots);
+// Bilinear REPEAT footprint of a sample in a map: the first texel of its two rows, whether the second column
+// wraps around (then the rows' first texels are the second column), and the four weights.
+struct Taps {
+    uint32_t row[2], x;
+    bool wraps;
+    float w[4];
+};
+__device__ inline Taps taps_of(const TexGPU& t, float u, float v) {
+    const float x = u * float(t.width) - 0.5f, y = v * float(t.height) - 0.5f;
+    const float fx = floorf(x), fy = floorf(y), ax = x - fx, ay = y - fy;
+    const int x0 = int(fx), y0 = int(fy), w = int(t.width), h = int(t.height);
+    const uint32_t xa = uint32_t(wrap_coord(x0, w, 2u));
+    const uint32_t ya = uint32_t(wrap_coord(y0, h, 2u)), yb = ya + 1u == t.height ? 0u : ya + 1u;
+    return {{ya * t.width, yb * t.width}, xa, xa + 1u == t.width, {(1 - ax) * (1 - ay), ax * (1 - ay), (1 - ax) * ay, ax * ay}};
+}
 
-    uint32_t slot, rx, ry, R;
+// The training target at (u, v), nm_target's value for the maps a decoded material has (four-channel
+// albedo, two-channel normal and metallic-roughness), in two parts: the texels -- the two of a row in
+// one load unless the footprint wraps around -- and their mix through the byte tables in LDS (lut[0]
+// UNORM, lut[1] sRGB).
+struct StepTexels {
+    uint32_t a[4], n[4], m[4];
+    float wa[4], wn[4], wm[4];
+};
+template <class T>
+__device__ inline void row_pair(const uint8_t* map, const Taps& t, int row, uint32_t& first, uint32_t& second) {
+    const T* p = reinterpret_cast<const T*>(map) + t.row[row];
+    struct __attribute__((packed)) Pair {
+        T a, b;
+    };
+    if (t.wraps) {
+        first = p[t.x];
+        second = p[0];
+    } else {
+        const Pair q = *reinterpret_cast<const Pair*>(p + t.x);
+        first = q.a;
+        second = q.b;
+    }
+}
+__device__ inline StepTexels step_texels(const uint8_t* texels, const TexGPU& ta, const TexGPU& tn, const TexGPU& tm,
+                                         float u, float v) {
+    const Taps a = taps_of(ta, u, v);  // maps of one extent (a uniform test) share their footprint
+    Taps n = a, m = a;
+    if (tn.width != ta.width || tn.height != ta.height) n = taps_of(tn, u, v);
+    if (tm.width != ta.width || tm.height != ta.height) m = taps_of(tm, u, v);
+    StepTexels p;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        row_pair<uint32_t>(texels + ta.offset, a, k, p.a[2 * k], p.a[2 * k + 1]);
+        row_pair<uint16_t>(texels + tn.offset, n, k, p.n[2 * k], p.n[2 * k + 1]);
+        row_pair<uint16_t>(texels + tm.offset, m, k, p.m[2 * k], p.m[2 * k + 1]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        p.wa[k] = a.w[k];
+        p.wn[k] = n.w[k];
+        p.wm[k] = m.w[k];
+    }
+    return p;
+}
+__device__ inline void step_target(const StepTexels& p, const TexGPU& ta, const TexGPU& tn, const TexGPU& tm,
+                                   const float (*lut)[256], float (&out)[kNmOut]) {
+    const float *la = lut[ta.srgb ? 1 : 0], *ln = lut[tn.srgb ? 1 : 0], *lm = lut[tm.srgb ? 1 : 0];
+    const auto mix = [](const float (&w)[4], const uint32_t (&t)[4], uint32_t c, const float* l) {
+        const uint32_t s = 8 * c;  // sample_tex's order and roundings
+        return fmaf(w[3], l[(t[3] >> s) & 0xffu], fmaf(w[2], l[(t[2] >> s) & 0xffu],
+                    fmaf(w[0], l[(t[0] >> s) & 0xffu], mul_rn(w[1], l[(t[1] >> s) & 0xffu]))));
+    };
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) out[c] = mix(p.wa, p.a, c, la);
+#pragma unroll
+    for (uint32_t c = 0; c < 2; ++c) {
+        out[3 + c] = mix(p.wn, p.n, c, ln);
+        out[5 + c] = mix(p.wm, p.m, c, lm);
+    }
+}
+
+// The MLP of a step as outer products: v_mfma_f32_4x4x1 with its A block broadcast adds w[0..3] * x to four
+// accumulators of every lane, w the four words of one 4-lane block and x the lane's own value -- so a
+// lane keeps its own sample throughout, nothing moves between lanes, the arithmetic is FP32 and the
+// weights are 19 registers.  An instruction takes 8 cycles where four multiply-adds take 16.
+// Weight word q of a table (block q % 16 of register q / 16) holds rows 4 (q % G) .. +3 of column q / G,
+// G groups of four rows; columns run over the bias, then the inputs (forward tables), or the outputs
+// of the layer (backward tables).
+__device__ inline f32x4 mfma_outer(float w, float x, f32x4 acc, int block) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    switch (block) {  // the block is an immediate
+#define RSY_OUTER(b) case b: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, x, acc, 4, b, 0)
+        RSY_OUTER(0); RSY_OUTER(1); RSY_OUTER(2); RSY_OUTER(3); RSY_OUTER(4); RSY_OUTER(5); RSY_OUTER(6); RSY_OUTER(7);
+        RSY_OUTER(8); RSY_OUTER(9); RSY_OUTER(10); RSY_OUTER(11); RSY_OUTER(12); RSY_OUTER(13); RSY_OUTER(14);
+        default: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, x, acc, 4, 15, 0);
+#undef RSY_OUTER
+    }
+#else
+    return acc;
+#endif
+}
+// The tables live in device memory in this form (one coalesced load a register): k_nm_mlp writes a
+// parameter's words after its update, k_nm_tables all of them before the first step.
+constexpr int kTabF1 = 0, kTabF2 = 6, kTabR2 = 11, kTabR1 = 15;  // [b1 | W1] and [b2 | W2] forward; W2 by hidden unit, W1 by latent channel
+static_assert(kTabR1 + 4 == kNmStepTables, "table registers");
+// Table words of parameter g (at most two).
+struct TableWords {
+    uint32_t n, at[2];
+};
+__host__ __device__ inline uint32_t table_word(int tab, uint32_t groups, uint32_t column, uint32_t row) {
+    const uint32_t q = column * groups + row / 4u;
+    return (uint32_t(tab) + q / 16u) * 64u + (q % 16u) * 4u + row % 4u;
+}
+__host__ __device__ inline TableWords table_words(uint32_t g) {
+    if (g < uint32_t(kNmB1)) {
+        const uint32_t j = g / kNmIn, k = g % kNmIn;
+        return {k < uint32_t(kNmCh) ? 2u : 1u, {table_word(kTabF1, 8, k + 1, j), table_word(kTabR1, 2, j, k)}};
+    }
+    if (g < uint32_t(kNmW2)) return {1u, {table_word(kTabF1, 8, 0, g - kNmB1), 0u}};
+    if (g < uint32_t(kNmB2)) {
+        const uint32_t c = (g - kNmW2) / kNmHidden, j = (g - kNmW2) % kNmHidden;
+        return {2u, {table_word(kTabF2, 2, j + 1, c), table_word(kTabR2, 8, c, j)}};
+    }
+    return {1u, {table_word(kTabF2, 2, 0, g - kNmB2), 0u}};
+}
+__device__ inline void write_table(float* tables, const TableWords& w, float x) {
+    tables[w.at[0]] = x;
+    if (w.n > 1) tables[w.at[1]] = x;
+}
+// (the words of no parameter stay the zeros the buffer was allocated with)
+__global__ __launch_bounds__(256) void k_nm_tables(const float* mlp, float* tables) {
+    const uint32_t g = blockIdx.x * 256 + threadIdx.x;
+    if (g < uint32_t(kNmParams)) write_table(tables, table_words(g), mlp[g]);
+}
+
+// One training step's samples: a workgroup per region; a thread of its first four waves per sample, the
+// other four hold the region's cells.
+//
+// A step has 65,536 samples by default: one sample wave on each of the chip's 1,024 SIMDs, so the kernel's
+// time is the length of one wave's chain: the step counter, the slot's map records, the texels (each
+// launch starts with a cold L2: 2,000 cycles a hop), the MLP, its gradient.
+// - Loads that depend on nothing else go out together at the start, the texels in pairs; the cell waves
+//   load the region's Adam state, whose latents the samples read from LDS.
+// - The MLP runs in registers on the matrix cores (its weights were read from LDS, one wait per hidden unit).
+// - Its gradient, a product over the samples, is one matrix instruction per sample and wave from
+//   records in LDS: 256 multiply-adds in sample order for every parameter, as the scalar loops had it
+//   (three dot products of 256 LDS pairs a thread, 20,000 cycles), 29 cycles apart.
+// - Latent gradients were 32 LDS float atomics a sample (20,000 cycles): the samples are sorted by cell
+//   while their texels are on the way, and the cell waves sum them and apply Adam beside the MLP gradient.
+// 65,536 samples of 16 materials: 47 us before, 18 us; the MLP's update 6.2 and 5.3 us.
+template <bool kExplicit>
+__global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
+    constexpr uint32_t kMaxCells = kMaxR * kMaxR, kCellsPerThread = kMaxCells / 256;
+    __shared__ __align__(16) float rec_s[256 * kRec];
+    __shared__ __align__(16) float4 lat_s[2 * kMaxCells];        // the region's latents, 8 a cell
+    __shared__ uint32_t count_s[kMaxCells], first_s[kMaxCells];  // samples per base cell and their first entry in order_s
+    __shared__ uint16_t order_s[256];                            // the chunk's samples by base cell
+    __shared__ uint32_t scan_s[kStepThreads / 64];
+    __shared__ float sum_s[kNmParamsPad];
+    __shared__ float lut[2][256];
+    __shared__ float red_s[kStepThreads / 64];
+    // waves 0..3 take the samples, waves 4..7 the region's cells
+    const uint32_t lane = threadIdx.x & 63u, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+    const bool sampler = wave < 4;
+    const uint32_t tid = threadIdx.x & 255u;
+    const uint32_t step = kExplicit ? 0u : *T.step + T.step_ahead;
+    const uint32_t L = T.L, Lm = L - 1;
+    const float inv_L = 1.f / float(L);  // exact: a power of two
+    float W[kNmStepTables] = {};
+    if (sampler)
+#pragma unroll
+        for (int v = 0; v < kNmStepTables; ++v) W[v] = T.tables[v * 64 + lane];
+
+    uint32_t slot, rx, ry, R, log2R;
     if (kExplicit) {
         slot = blockIdx.x;
         rx = ry = 0;
         R = L;
+        log2R = T.log2L;
     } else {
-        R = 1u << T.log2R;
-        const uint32_t log2rx = T.log2L - T.log2R;
+        log2R = T.log2R;
+        R = 1u << log2R;
+        const uint32_t log2rx = T.log2L - log2R;
         const uint32_t rpm = 1u << (2 * log2rx);  // regions per grid
         const uint64_t n_regions = uint64_t(T.n_slots) * rpm;
         const uint64_t r = (uint64_t(step) * T.n_wg + blockIdx.x) % n_regions;
@@ -85,16 +267,45 @@ __global__ __launch_bounds__(256) void k_nm_step(NmTrainLaunch T) {
         rx = (reg & ((1u << log2rx) - 1)) * R + ox;
         ry = (reg >> log2rx) * R + oy;
     }
-    const uint32_t n_el = R * R * kNmCh;
-    const size_t grid_base = size_t(slot) * L * L * kNmCh;
-    for (uint32_t i = tid; i < n_el; i += 256) {
-        const uint32_t c = i & 7u, cell = i >> 3, cx = cell % R, cy = cell / R;
-        const size_t g = grid_base + (size_t((ry + cy) & Lm) * L + ((rx + cx) & Lm)) * kNmCh + c;
-        lat_s[i] = T.lat[g];
-        grad_s[i] = 0.f;
+    const uint32_t cells = R * R;
+    const size_t grid_base = size_t(slot) * L * L;
+    auto cell_of = [&](uint32_t cx, uint32_t cy) { return grid_base + size_t((ry + cy) & Lm) * L + ((rx + cx) & Lm); };
+    TexGPU ta{}, tn{}, tm{};
+    float4 adam[6] = {};  // a cell wave: the Adam state of the thread's first cell, and the step's factors
+    float bc1 = 1.f, bc2 = 1.f, lr = 0.f;
+    if (sampler) {
+        ta = T.maps[3 * slot];
+        tn = T.maps[3 * slot + 1];
+        tm = T.maps[3 * slot + 2];
+    } else {
+        const float srgb = T.srgb_lut[tid];
+        if (!kExplicit && tid < cells) {
+            const size_t g = 2 * cell_of(tid & (R - 1), tid >> log2R);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                adam[k] = reinterpret_cast<const float4*>(T.lat)[g + k];
+                adam[2 + k] = reinterpret_cast<const float4*>(T.lat_m)[g + k];
+                adam[4 + k] = reinterpret_cast<const float4*>(T.lat_v)[g + k];
+            }
+        }
+        for (uint32_t i = tid; i < cells; i += 256) {
+            count_s[i] = 0u;
+            if (!kExplicit && i < 256) {
+                lat_s[2 * i] = adam[0];
+                lat_s[2 * i + 1] = adam[1];
+            } else {
+                const size_t g = 2 * cell_of(i & (R - 1), i >> log2R);
+                lat_s[2 * i] = reinterpret_cast<const float4*>(T.lat)[g];
+                lat_s[2 * i + 1] = reinterpret_cast<const float4*>(T.lat)[g + 1];
+            }
+        }
+        lut[0][tid] = float(tid) * (1.0f / 255.0f);
+        lut[1][tid] = srgb;
+        const float t = float(step + 1);
+        bc1 = 1.f - powf(T.beta1, t);
+        bc2 = 1.f - powf(T.beta2, t);
+        lr = T.lr_lat * lr_factor(step, T.decay_steps);
     }
-    for (uint32_t i = tid; i < uint32_t(kNmParamsPad); i += 256) w_s[i] = T.mlp[i];
-    __syncthreads();
 
     uint32_t n_samples, s_base = 0;
     if (kExplicit) {
@@ -103,22 +314,27 @@ __global__ __launch_bounds__(256) void k_nm_step(NmTrainLaunch T) {
     } else {
         n_samples = T.spw;
     }
-    const NmSlot S = slots[slot];
     const uint64_t skey = mix64(T.seed + 0x632BE59BD9B4E019ull * (uint64_t(step) + 1)) + (uint64_t(blockIdx.x) << 32);
-    float acc[3] = {0.f, 0.f, 0.f};
+    float* const rec = rec_s + tid * kRec;
+    // the lane's block of the gradient products: its row operand and column operand in a record
+    const uint32_t blk = wave * 16u + (lane >> 2), blk2 = blk - kGradBlocks1;
+    const bool first_layer = blk < kGradBlocks1, bias2 = blk >= kGradBlocks1 + kGradBlocks2;
+    const uint32_t row_at = (first_layer ? kRecDh + 4u * (blk / 3u) : bias2 ? kRecIn + 8u : kRecH + 4u * (blk2 / 2u)) + (lane & 3u);
+    const uint32_t col_at = (first_layer ? kRecIn + 4u * (blk % 3u) : kRecDo + 4u * (blk2 % 2u)) + (lane & 3u);
+    f32x4 grad = {};                          // of the lane's block
+    float grad_lat[kCellsPerThread][kNmCh] = {};  // of the thread's cells tid, tid + 256, ...
     float loss = 0.f;
-    const float* W1 = w_s + kNmW1;
-    const float* B1 = w_s + kNmB1;
-    const float* W2 = w_s + kNmW2;
-    const float* B2 = w_s + kNmB2;
     for (uint32_t base = 0; base < n_samples; base += 256) {
         const uint32_t q = base + tid;
-        float* rec = rec_s + tid * kRec;
-        if (q < n_samples) {
-            float ax, ay, tgt[kNmOut];
-            uint32_t i0, i1, j0, j1;
+        const bool live = sampler && q < n_samples;
+        float tgt[kNmOut] = {}, ax = 0.f, ay = 0.f;
+        uint32_t i0 = 0, i1 = 0, j0 = 0, j1 = 0;
+        StepTexels px{};
+        if (live) {
+            float u, v;
             if (kExplicit) {
-                const float u = T.ex_uv[2 * size_t(s_base + q)], v = T.ex_uv[2 * size_t(s_base + q) + 1];
+                u = T.ex_uv[2 * size_t(s_base + q)];
+                v = T.ex_uv[2 * size_t(s_base + q) + 1];
                 const float x = u * float(L) - 0.5f, y = v * float(L) - 0.5f;
                 const float fx = floorf(x), fy = floorf(y);
                 ax = x - fx;
@@ -127,157 +343,310 @@ __global__ __launch_bounds__(256) void k_nm_step(NmTrainLaunch T) {
                 j0 = uint32_t(int(fy)) & Lm;
                 i1 = (i0 + 1) & Lm;
                 j1 = (j0 + 1) & Lm;
-#pragma unroll
-                for (int c = 0; c < kNmOut; ++c) tgt[c] = T.ex_target[kNmOut * size_t(s_base + q) + c];
             } else {
-                const uint64_t h = mix64(skey + q);
-                const float xl = unit24(uint32_t(h)) * float(R - 1), yl = unit24(uint32_t(h >> 32)) * float(R - 1);
+                const uint64_t hh = mix64(skey + q);
+                const float sx = unit24(uint32_t(hh)), sy = unit24(uint32_t(hh >> 32)), span = float(R - 1);
+                const float xl = mul_rn(sx, span), yl = mul_rn(sy, span);
                 i0 = min(uint32_t(xl), R - 2);
                 j0 = min(uint32_t(yl), R - 2);
                 ax = xl - float(i0);
                 ay = yl - float(j0);
+                u = (fmaf(sx, span, float(rx)) + 0.5f) * inv_L;
+                v = (fmaf(sy, span, float(ry)) + 0.5f) * inv_L;
                 i1 = i0 + 1;
                 j1 = j0 + 1;
-                const float u = (float(rx) + xl + 0.5f) / float(L), v = (float(ry) + yl + 0.5f) / float(L);
-                nm_target(T.texels, T.textures, S, u, v, T.srgb_lut, tgt);
             }
-            const float w00 = (1.f - ax) * (1.f - ay), w10 = ax * (1.f - ay), w01 = (1.f - ax) * ay, w11 = ax * ay;
-            const uint32_t c00 = (j0 * R + i0) * kNmCh, c10 = (j0 * R + i1) * kNmCh;
-            const uint32_t c01 = (j1 * R + i0) * kNmCh, c11 = (j1 * R + i1) * kNmCh;
-            float in[kNmIn];
+            if (kExplicit) {
 #pragma unroll
-            for (int c = 0; c < kNmCh; ++c)
-                in[c] = w00 * lat_s[c00 + c] + w10 * lat_s[c10 + c] + w01 * lat_s[c01 + c] + w11 * lat_s[c11 + c];
-            in[8] = 1.f - fabsf(2.f * ax - 1.f);
-            in[9] = 1.f - fabsf(2.f * ay - 1.f);
-            // forward: hidden activations go straight to the sample's LDS record
-#pragma unroll 2
-            for (int j = 0; j < kNmHidden; ++j) {
-                float z = B1[j];
-#pragma unroll
-                for (int k = 0; k < kNmIn; ++k) z += W1[j * kNmIn + k] * in[k];
-                rec[kRecH + j] = fmaxf(z, 0.f);
+                for (int c = 0; c < kNmOut; ++c) tgt[c] = T.ex_target[kNmOut * size_t(s_base + q) + c];
+            } else {
+                px = step_texels(T.texels, ta, tn, tm, u, v);
             }
-            float dout[kNmOut];
+        }
+        __syncthreads();  // counts cleared, tables written, the last chunk's records read
+        // the chunk's samples sorted by base cell while their texels and cells are on the way
+        const uint32_t bin = j0 * R + i0;
+        const uint32_t rank = live ? atomicAdd(&count_s[bin], 1u) : 0u;
+        __syncthreads();
+        {
+            uint32_t n[kCellsPerThread] = {}, mine = 0, total;
+#pragma unroll
+            for (uint32_t k = 0; k < kCellsPerThread; ++k) {
+                const uint32_t c = tid * kCellsPerThread + k;
+                if (!sampler && c < cells) n[k] = count_s[c];
+                mine += n[k];
+            }
+            uint32_t at = block_exclusive_scan(mine, scan_s, total);
+#pragma unroll
+            for (uint32_t k = 0; k < kCellsPerThread; ++k) {
+                const uint32_t c = tid * kCellsPerThread + k;
+                if (!sampler && c < cells) first_s[c] = at;
+                at += n[k];
+            }
+        }
+        __syncthreads();
+        if (sampler) {
+            if (live) order_s[first_s[bin] + rank] = uint16_t(tid);
+            float in[kNmIn] = {};
+            if (live) {
+                const float w00 = (1.f - ax) * (1.f - ay), w10 = ax * (1.f - ay), w01 = (1.f - ax) * ay, w11 = ax * ay;
+                const float4 *q00 = lat_s + 2 * (j0 * R + i0), *q10 = lat_s + 2 * (j0 * R + i1);
+                const float4 *q01 = lat_s + 2 * (j1 * R + i0), *q11 = lat_s + 2 * (j1 * R + i1);
+                const float4 c00[2] = {q00[0], q00[1]}, c10[2] = {q10[0], q10[1]};
+                const float4 c01[2] = {q01[0], q01[1]}, c11[2] = {q11[0], q11[1]};
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    in[4 * k + 0] = w00 * c00[k].x + w10 * c10[k].x + w01 * c01[k].x + w11 * c11[k].x;
+                    in[4 * k + 1] = w00 * c00[k].y + w10 * c10[k].y + w01 * c01[k].y + w11 * c11[k].y;
+                    in[4 * k + 2] = w00 * c00[k].z + w10 * c10[k].z + w01 * c01[k].z + w11 * c11[k].z;
+                    in[4 * k + 3] = w00 * c00[k].w + w10 * c10[k].w + w01 * c01[k].w + w11 * c11[k].w;
+                }
+                in[8] = 1.f - fabsf(2.f * ax - 1.f);
+                in[9] = 1.f - fabsf(2.f * ay - 1.f);
+                if (!kExplicit) step_target(px, ta, tn, tm, lut, tgt);
+            }
+            // forward and backward in every lane (a lane without a sample has zero features and zero dL/dout)
+            f32x4 acc[8], o2[2] = {}, dz[8], din[2] = {};
+#pragma unroll
+            for (int g = 0; g < 8; ++g) acc[g] = mfma_outer(W[kTabF1 + g / 16], 1.f, f32x4{}, g % 16);
+#pragma unroll
+            for (int k = 0; k < kNmIn; ++k)
+#pragma unroll
+                for (int g = 0; g < 8; ++g) acc[g] = mfma_outer(W[kTabF1 + (8 * k + 8 + g) / 16], in[k], acc[g], (8 * k + 8 + g) % 16);
+            float h[kNmHidden], dh[kNmHidden], dout[kNmOut];
+#pragma unroll
+            for (int j = 0; j < kNmHidden; ++j) h[j] = fmaxf(acc[j / 4][j % 4], 0.f);
+#pragma unroll
+            for (int g = 0; g < 2; ++g) o2[g] = mfma_outer(W[kTabF2], 1.f, f32x4{}, g);
+#pragma unroll
+            for (int j = 0; j < kNmHidden; ++j)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) o2[g] = mfma_outer(W[kTabF2 + (2 * j + 2 + g) / 16], h[j], o2[g], (2 * j + 2 + g) % 16);
 #pragma unroll
             for (int c = 0; c < kNmOut; ++c) {
-                float o = B2[c];
-#pragma unroll 4
-                for (int j = 0; j < kNmHidden; ++j) o += W2[c * kNmHidden + j] * rec[kRecH + j];
-                const float d = o - tgt[c];
+                const float d = live ? o2[c / 4][c % 4] - tgt[c] : 0.f;
                 loss += d * d;
                 dout[c] = 2.f * d * T.inv_norm;
-                rec[kRecDo + c] = dout[c];
             }
             // backward: dL/dhidden (ReLU mask), dL/dfeatures for the 8 latent channels
-            float din[kNmCh] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-            for (int j = 0; j < kNmHidden; ++j) {
-                float g = 0.f;
 #pragma unroll
-                for (int c = 0; c < kNmOut; ++c) g += W2[c * kNmHidden + j] * dout[c];
-                const float dh = rec[kRecH + j] > 0.f ? g : 0.f;
-                rec[kRecDh + j] = dh;
+            for (int g = 0; g < 8; ++g) dz[g] = mfma_outer(W[kTabR2], dout[0], f32x4{}, g);
 #pragma unroll
-                for (int c = 0; c < kNmCh; ++c) din[c] += W1[j * kNmIn + c] * dh;
+            for (int c = 1; c < kNmOut; ++c)
+#pragma unroll
+                for (int g = 0; g < 8; ++g) dz[g] = mfma_outer(W[kTabR2 + (8 * c + g) / 16], dout[c], dz[g], (8 * c + g) % 16);
+#pragma unroll
+            for (int j = 0; j < kNmHidden; ++j) dh[j] = h[j] > 0.f ? dz[j / 4][j % 4] : 0.f;
+#pragma unroll
+            for (int j = 0; j < kNmHidden; ++j)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) din[g] = mfma_outer(W[kTabR1 + (2 * j + g) / 16], dh[j], din[g], (2 * j + g) % 16);
+            // the sample's record (zeros past the last sample: no contribution)
+#pragma unroll
+            for (int k = 0; k < kNmHidden; k += 4) {
+                *reinterpret_cast<float4*>(rec + kRecDh + k) = make_float4(dh[k], dh[k + 1], dh[k + 2], dh[k + 3]);
+                *reinterpret_cast<float4*>(rec + kRecH + k) = make_float4(h[k], h[k + 1], h[k + 2], h[k + 3]);
             }
-#pragma unroll
-            for (int c = 0; c < kNmCh; ++c) {
-                atomicAdd(&grad_s[c00 + c], w00 * din[c]);
-                atomicAdd(&grad_s[c10 + c], w10 * din[c]);
-                atomicAdd(&grad_s[c01 + c], w01 * din[c]);
-                atomicAdd(&grad_s[c11 + c], w11 * din[c]);
-            }
-#pragma unroll
-            for (int k = 0; k < kNmIn; ++k) rec[kRecIn + k] = in[k];
+            *reinterpret_cast<float4*>(rec + kRecIn) = make_float4(in[0], in[1], in[2], in[3]);
+            *reinterpret_cast<float4*>(rec + kRecIn + 4) = make_float4(in[4], in[5], in[6], in[7]);
+            *reinterpret_cast<float4*>(rec + kRecIn + 8) = make_float4(in[8], in[9], 1.f, ax);
+            *reinterpret_cast<float4*>(rec + kRecDo) = make_float4(dout[0], dout[1], dout[2], dout[3]);
+            *reinterpret_cast<float4*>(rec + kRecDo + 4) = make_float4(dout[4], dout[5], dout[6], ay);
+            *reinterpret_cast<f32x4*>(rec + kRecDl) = din[0];
+            *reinterpret_cast<f32x4*>(rec + kRecDl + 4) = din[1];
         }
         __syncthreads();
-        // MLP gradient components tid, tid + 256, tid + 512 over this chunk's samples
-        const uint32_t cnt = min(256u, n_samples - base);
+        // each wave its sixteen blocks over all records, one sample an instruction: every gradient is the
+        // multiply-add chain over the samples in their order, whatever the wave that runs it.  A batch of
+        // operands is read while the last one goes through the chain.
+        if (wave < kGradWaves) {
+            constexpr uint32_t kBatch = 16;
+            const float* const pr = rec_s + min(row_at, uint32_t(kRec - 1));
+            const float* const pc = rec_s + min(col_at, uint32_t(kRec - 1));
+            f32x4 s = {};
+            const uint32_t cnt = min(256u, n_samples - base);  // records from cnt on are zeros
+            float a[kBatch], b[kBatch];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const uint32_t g = tid + 256u * a;
-            if (g >= uint32_t(kNmParams)) continue;
-            float s = 0.f;
-            if (g < uint32_t(kNmB1)) {
-                const uint32_t j = g / kNmIn, k = g % kNmIn;
-                for (uint32_t r = 0; r < cnt; ++r) s += rec_s[r * kRec + kRecDh + j] * rec_s[r * kRec + kRecIn + k];
-            } else if (g < uint32_t(kNmW2)) {
-                const uint32_t j = g - kNmB1;
-                for (uint32_t r = 0; r < cnt; ++r) s += rec_s[r * kRec + kRecDh + j];
-            } else if (g < uint32_t(kNmB2)) {
-                const uint32_t c = (g - kNmW2) / kNmHidden, j = (g - kNmW2) % kNmHidden;
-                for (uint32_t r = 0; r < cnt; ++r) s += rec_s[r * kRec + kRecDo + c] * rec_s[r * kRec + kRecH + j];
-            } else {
-                const uint32_t c = g - kNmB2;
-                for (uint32_t r = 0; r < cnt; ++r) s += rec_s[r * kRec + kRecDo + c];
+            for (uint32_t k = 0; k < kBatch; ++k) {
+                a[k] = pr[k * kRec];
+                b[k] = pc[k * kRec];
             }
-            acc[a] += s;
+            for (uint32_t r = 0; r < cnt; r += kBatch) {
+                float na[kBatch], nb[kBatch];
+                const uint32_t next = min(r + kBatch, 256u - kBatch);
+#pragma unroll
+                for (uint32_t k = 0; k < kBatch; ++k) {
+                    na[k] = pr[(next + k) * kRec];
+                    nb[k] = pc[(next + k) * kRec];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < kBatch; ++k) s = __builtin_amdgcn_mfma_f32_4x4x1f32(a[k], b[k], s, 0, 0, 0);
+#pragma unroll
+                for (uint32_t k = 0; k < kBatch; ++k) {
+                    a[k] = na[k];
+                    b[k] = nb[k];
+                }
+            }
+            grad += s;
+        }
+        // meanwhile the cell waves gather: a cell is a corner of four base cells' samples (a base cell in the last
+        // column or row has no samples in a region, and wraps around in a whole grid); the four lists are
+        // walked as one, the next sample's place read ahead
+        if (!sampler) {
+#pragma unroll
+            for (uint32_t k = 0; k < kCellsPerThread; ++k) {
+                const uint32_t cell = tid + 256u * k;
+                if (cell >= cells) break;
+                const uint32_t cx = cell & (R - 1), cy = cell >> log2R;
+                uint32_t end[4], at[4], n = 0;
+#pragma unroll
+                for (uint32_t c = 0; c < 4; ++c) {
+                    const uint32_t from = ((cy - (c >> 1)) & (R - 1)) * R + ((cx - (c & 1u)) & (R - 1));
+                    at[c] = first_s[from] - n;  // entry i of the joint list: at[c] + i for i in [end[c - 1], end[c])
+                    n += count_s[from];
+                    end[c] = n;
+                }
+                const auto place = [&](uint32_t i) {
+                    const uint32_t a = i < end[0] ? at[0] : i < end[1] ? at[1] : i < end[2] ? at[2] : at[3];
+                    return uint32_t(order_s[min(a + i, 255u)]) * kRec;
+                };
+                uint32_t o = n ? place(0) : 0u;
+                for (uint32_t i = 0; i < n; ++i) {
+                    const float* r = rec_s + o;
+                    const float x = r[kRecAx], y = r[kRecAy];
+                    const f32x4 d0 = *reinterpret_cast<const f32x4*>(r + kRecDl), d1 = *reinterpret_cast<const f32x4*>(r + kRecDl + 4);
+                    o = place(i + 1);
+                    const bool right = (i >= end[0] && i < end[1]) || i >= end[2], low = i >= end[1];
+                    const float w = (right ? x : 1.f - x) * (low ? y : 1.f - y);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        grad_lat[k][c] += w * d0[c];
+                        grad_lat[k][4 + c] += w * d1[c];
+                    }
+                }
+            }
         }
         __syncthreads();
+        if (!sampler)
+            for (uint32_t i = tid; i < cells; i += 256) count_s[i] = 0u;
     }
-    const float loss_sum = block_sum(loss, red_s);
-    // partial sums, parameter-major: partial[g * n_wg + workgroup]
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const uint32_t g = tid + 256u * a;
-        if (g < uint32_t(kNmParams)) T.partial[size_t(g) * T.n_wg + blockIdx.x] = acc[a];
-    }
-    if (tid == 0) T.partial[size_t(kNmParams) * T.n_wg + blockIdx.x] = loss_sum;
-
     // latents of the region: gradient out (explicit mode) or Adam
-    const float t = float(step + 1);
-    const float bc1 = 1.f - powf(T.beta1, t), bc2 = 1.f - powf(T.beta2, t);
-    const float lr = T.lr_lat * lr_factor(step, T.decay_steps);
-    for (uint32_t i = tid; i < n_el; i += 256) {
-        const uint32_t c = i & 7u, cell = i >> 3, cx = cell % R, cy = cell / R;
-        const size_t g = grid_base + (size_t((ry + cy) & Lm) * L + ((rx + cx) & Lm)) * kNmCh + c;
-        const float gr = grad_s[i];
-        if (kExplicit) {
-            T.ex_grad_lat[g] = gr;
-        } else {
-            const float m = T.beta1 * T.lat_m[g] + (1.f - T.beta1) * gr;
-            const float v = T.beta2 * T.lat_v[g] + (1.f - T.beta2) * gr * gr;
-            T.lat_m[g] = m;
-            T.lat_v[g] = v;
-            T.lat[g] = lat_s[i] - lr * (m / bc1) / (sqrtf(v / bc2) + T.eps);
+    if (!sampler) {
+#pragma unroll
+        for (uint32_t k = 0; k < kCellsPerThread; ++k) {
+            const uint32_t cell = tid + 256u * k;
+            if (cell >= cells) break;
+            const size_t g = 2 * cell_of(cell & (R - 1), cell >> log2R);
+            if (!kExplicit && k > 0)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    adam[i] = reinterpret_cast<const float4*>(T.lat)[g + i];
+                    adam[2 + i] = reinterpret_cast<const float4*>(T.lat_m)[g + i];
+                    adam[4 + i] = reinterpret_cast<const float4*>(T.lat_v)[g + i];
+                }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const float* gr = grad_lat[k] + 4 * i;
+                if (kExplicit) {
+                    reinterpret_cast<float4*>(T.ex_grad_lat)[g + i] = make_float4(gr[0], gr[1], gr[2], gr[3]);
+                } else {
+                    float4 &x = adam[i], &m = adam[2 + i], &v = adam[4 + i];
+                    adam_step(x.x, m.x, v.x, gr[0], T, lr, bc1, bc2);
+                    adam_step(x.y, m.y, v.y, gr[1], T, lr, bc1, bc2);
+                    adam_step(x.z, m.z, v.z, gr[2], T, lr, bc1, bc2);
+                    adam_step(x.w, m.w, v.w, gr[3], T, lr, bc1, bc2);
+                    reinterpret_cast<float4*>(T.lat)[g + i] = x;
+                    reinterpret_cast<float4*>(T.lat_m)[g + i] = m;
+                    reinterpret_cast<float4*>(T.lat_v)[g + i] = v;
+                }
+            }
         }
     }
+    // the workgroup's sums: a lane holds rows 0..3 of its block's column lane % 4
+    if (sampler && blk < kGradBlocks) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t col = 4u * (first_layer ? blk % 3u : blk2 % 2u) + (lane & 3u);
+            const uint32_t j = 4u * (first_layer ? blk / 3u : blk2 / 2u) + i;
+            if (first_layer) {
+                if (col < uint32_t(kNmIn)) sum_s[kNmW1 + j * kNmIn + col] = grad[i];
+                else if (col == uint32_t(kNmIn)) sum_s[kNmB1 + j] = grad[i];
+            } else if (col < uint32_t(kNmOut)) {
+                if (!bias2) sum_s[kNmW2 + col * kNmHidden + j] = grad[i];
+                else if (i == uint32_t(kNmIn) - 8u) sum_s[kNmB2 + col] = grad[i];
+            }
+        }
+    }
+    const float loss_sum = block_sum(loss, red_s);  // synchronises
+    if (threadIdx.x == 0) sum_s[kNmParams] = loss_sum;
+    __syncthreads();
+    // workgroup-major: partial[workgroup * 584 + g], the loss last
+    for (uint32_t g = threadIdx.x; g < uint32_t(kNmParamsPad); g += kStepThreads) T.partial[size_t(blockIdx.x) * kNmParamsPad + g] = sum_s[g];
 }
 
-// One wave per MLP parameter (and one for the loss): sums that parameter's per-workgroup partials
-// (lane-strided, then a fixed-order wave reduction), then Adam (or, in explicit mode, writes the
-// summed gradient) and records the step's loss.
+// The MLP's update: a block per 64 parameters (one a lane), its 16 waves summing the workgroups'
+// partials -- coalesced rows, a wave's rows in flight together -- in a fixed order: 64 strided sums (the
+// workgroups i, i + 64, ... of sum i), then those pairwise, i with i + 32, then + 16, + 8, ... -- then Adam (or, in explicit
+// mode, the summed gradient) and the step's loss.  6.2 us as one wave per parameter over a
+// parameter-major table, 5.3 us.
+constexpr uint32_t kMlpWaves = 16;
 template <bool kExplicit>
-__global__ __launch_bounds__(256) void k_nm_mlp(NmTrainLaunch T) {
-    const uint32_t g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (g >= uint32_t(kNmParamsPad)) return;
-    const uint32_t step = kExplicit ? 0u : *T.step;
-    const float* P = T.partial + size_t(g) * T.n_wg;
-    float s = 0.f;
-    for (uint32_t b = lane; b < T.n_wg; b += 64) s += P[b];
+__global__ __launch_bounds__(64 * kMlpWaves) void k_nm_mlp(NmTrainLaunch T) {
+    __shared__ float sums[kMlpWaves][64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, g = blockIdx.x * 64 + lane;
+    const bool live = g < uint32_t(kNmParamsPad);
+    const uint32_t step = kExplicit ? 0u : *T.step + T.step_ahead;
+    float m = 0.f, v = 0.f, x = 0.f;
+    const TableWords words = table_words(min(g, uint32_t(kNmParams - 1)));
+    const bool update = !kExplicit && wave == 0 && g < uint32_t(kNmParams);
+    if (update) {
+        m = T.mlp_m[g];
+        v = T.mlp_v[g];
+        x = T.mlp[g];
+    }
+    float s4[4] = {};  // sums wave, wave + 16, wave + 32, wave + 48
+    if (live)
+        for (uint32_t b = wave; b < T.n_wg; b += 256) {
+            float p[4][4];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (lane != 0) return;
+            for (uint32_t k = 0; k < 4; ++k)
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const uint32_t wg = b + 64 * k + 16 * i;
+                    p[k][i] = wg < T.n_wg ? T.partial[size_t(wg) * kNmParamsPad + g] : 0.f;
+                }
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) s4[i] += p[k][i];
+        }
+    sums[wave][lane] = (s4[0] + s4[2]) + (s4[1] + s4[3]);
+#pragma unroll
+    for (uint32_t o = kMlpWaves / 2; o > 0; o >>= 1) {
+        __syncthreads();
+        if (wave < o) sums[wave][lane] += sums[wave + o][lane];
+    }
+    if (wave != 0 || !live) return;
+    const float s = sums[0][lane];
     if (kExplicit) {
         T.ex_grad_mlp[g] = s;
-    } else if (g < uint32_t(kNmParams)) {
+    } else if (update) {
         const float t = float(step + 1);
         const float bc1 = 1.f - powf(T.beta1, t), bc2 = 1.f - powf(T.beta2, t);
         const float lr = T.lr_mlp * lr_factor(step, T.decay_steps);
-        const float m = T.beta1 * T.mlp_m[g] + (1.f - T.beta1) * s;
-        const float v = T.beta2 * T.mlp_v[g] + (1.f - T.beta2) * s * s;
+        adam_step(x, m, v, s, T, lr, bc1, bc2);
         T.mlp_m[g] = m;
         T.mlp_v[g] = v;
-        T.mlp[g] -= lr * (m / bc1) / (sqrtf(v / bc2) + T.eps);
+        T.mlp[g] = x;
+        write_table(T.tables, words, x);
     } else if (T.loss_out && step >= T.loss_base && step - T.loss_base < T.loss_cap) {
         T.loss_out[step - T.loss_base] = s * T.inv_norm;  // mean squared error of the step
     }
 }
 
-// Advances the device step counter once every reader of this step has finished.
-__global__ void k_nm_advance(uint32_t* step) {
-    if (threadIdx.x == 0) *step += 1u;
+// Advances the device step counter by a batch of steps, once their readers have finished.
+__global__ void k_nm_advance(uint32_t* step, uint32_t steps) {
+    if (threadIdx.x == 0) *step += steps;
 }
 
 __global__ __launch_bounds__(256) void k_nm_init(NmInitLaunch I) {
@@ -551,17 +920,25 @@ hipError_t launch_nm_init(const NmInitLaunch& l, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_nm_step(const NmTrainLaunch& l, bool explicit_batch, hipStream_t s) {
-    if (explicit_batch) {
-        if (l.L > uint32_t(kMaxR)) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_nm_step<true>, dim3(l.n_slots), dim3(256), 0, s, l);
-        hipLaunchKernelGGL(k_nm_mlp<true>, dim3(kNmParamsPad / 4), dim3(256), 0, s, l);
-    } else {
-        if ((1u << l.log2R) > uint32_t(kMaxR) || l.log2R > l.log2L || l.log2R < 1) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_nm_step<false>, dim3(l.n_wg), dim3(256), 0, s, l);
-        hipLaunchKernelGGL(k_nm_mlp<false>, dim3(kNmParamsPad / 4), dim3(256), 0, s, l);
-        hipLaunchKernelGGL(k_nm_advance, dim3(1), dim3(64), 0, s, l.step);
+hipError_t launch_nm_gradient(const NmTrainLaunch& l, hipStream_t s) {
+    if (l.L > uint32_t(kMaxR)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_nm_step<true>, dim3(l.n_slots), dim3(kStepThreads), 0, s, l);
+    hipLaunchKernelGGL(k_nm_mlp<true>, dim3((kNmParamsPad + 63) / 64), dim3(64 * kMlpWaves), 0, s, l);
+    return hipGetLastError();
+}
+
+hipError_t launch_nm_tables(const NmTrainLaunch& l, hipStream_t s) {
+    hipLaunchKernelGGL(k_nm_tables, dim3((kNmParams + 255) / 256), dim3(256), 0, s, l.mlp, l.tables);
+    return hipGetLastError();
+}
+
+hipError_t launch_nm_steps(NmTrainLaunch l, uint32_t steps, hipStream_t s) {
+    if ((1u << l.log2R) > uint32_t(kMaxR) || l.log2R > l.log2L || l.log2R < 1) return hipErrorInvalidValue;
+    for (l.step_ahead = 0; l.step_ahead < steps; ++l.step_ahead) {
+        hipLaunchKernelGGL(k_nm_step<false>, dim3(l.n_wg), dim3(kStepThreads), 0, s, l);
+        hipLaunchKernelGGL(k_nm_mlp<false>, dim3((kNmParamsPad + 63) / 64), dim3(64 * kMlpWaves), 0, s, l);
     }
+    hipLaunchKernelGGL(k_nm_advance, dim3(1), dim3(64), 0, s, l.step, steps);
     return hipGetLastError();
 }
 

@@ -28,8 +28,8 @@ struct NeuralState {
     std::vector<uint32_t> block_base;  // evaluation tiles per slot (prefix, n_slots + 1)
     uint32_t max_tiles = 0;            // of the largest slot
     bool any_same = false, any_other = false;  // some slot's maps share one extent / differ in size
-    DevBuf slots_d, slot_of_d, active_d, block_base_d;
-    DevBuf lat, lat_m, lat_v, mlp, mlp_m, mlp_v, partial, step_d, loss_d, lat16, weights_d, eval_partial, eval_sum;
+    DevBuf slots_d, maps_d, slot_of_d, active_d, block_base_d;
+    DevBuf lat, lat_m, lat_v, mlp, mlp_m, mlp_v, tables, partial, step_d, loss_d, lat16, weights_d, eval_partial, eval_sum;
     DevBuf tmp[5];
     uint32_t n_wg = 0, spw = 0;
     uint32_t steps = 0;
@@ -130,11 +130,11 @@ NmTrainLaunch train_args(rsy_ctx* c, NeuralState* n) {
     T.mlp = n->mlp.as<float>();
     T.mlp_m = n->mlp_m.as<float>();
     T.mlp_v = n->mlp_v.as<float>();
+    T.tables = n->tables.as<float>();
     T.partial = n->partial.as<float>();
     T.step = n->step_d.as<uint32_t>();
-    T.slots = n->slots_d.p;
+    T.maps = n->maps_d.as<TexGPU>();
     T.n_slots = uint32_t(n->slots.size());
-    T.textures = c->tex_table.as<TexGPU>();
     T.texels = c->texels.as<uint8_t>();
     T.srgb_lut = c->srgb_lut.as<float>();
     T.L = n->L;
@@ -239,6 +239,7 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     HIP_TRY(c, hipEventCreate(&n->ev0), "event");
     HIP_TRY(c, hipEventCreate(&n->ev1), "event");
     HIP_TRY(c, n->slots_d.ensure(std::max<size_t>(1, ns) * sizeof(NmSlot)), "allocate decoder");
+    HIP_TRY(c, n->maps_d.ensure(std::max<size_t>(1, ns) * 3 * sizeof(TexGPU)), "allocate decoder");
     HIP_TRY(c, n->slot_of_d.ensure(std::max<size_t>(1, nm) * 4), "allocate decoder");
     HIP_TRY(c, n->active_d.ensure(std::max<size_t>(1, nm) * 4), "allocate decoder");
     HIP_TRY(c, n->block_base_d.ensure((ns + 1) * 4), "allocate decoder");
@@ -250,13 +251,20 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     HIP_TRY(c, n->mlp.ensure(kNmParamsPad * 4), "allocate decoder");
     HIP_TRY(c, n->mlp_m.ensure(kNmParamsPad * 4), "allocate decoder");
     HIP_TRY(c, n->mlp_v.ensure(kNmParamsPad * 4), "allocate decoder");
+    HIP_TRY(c, n->tables.ensure(kNmStepTables * 64 * 4), "allocate decoder");
     HIP_TRY(c, n->partial.ensure(size_t(std::max<uint32_t>(n->n_wg, std::max<uint32_t>(1, ns))) * kNmParamsPad * 4),
             "allocate decoder");
     HIP_TRY(c, n->step_d.ensure(4), "allocate decoder");
     HIP_TRY(c, n->weights_d.ensure(kNmWeightsBytes), "allocate decoder");
     HIP_TRY(c, n->eval_partial.ensure(size_t(std::max<uint32_t>(1, n->block_base[ns])) * 4), "allocate decoder");
     HIP_TRY(c, n->eval_sum.ensure(std::max<size_t>(1, ns) * 8), "allocate decoder");
-    if (ns) HIP_TRY(c, hipMemcpy(n->slots_d.p, n->slots.data(), ns * sizeof(NmSlot), hipMemcpyHostToDevice), "upload");
+    if (ns) {
+        std::vector<TexGPU> maps;
+        for (const NmSlot& sl : n->slots)
+            for (uint32_t k : {sl.albedo, sl.normal, sl.mr}) maps.push_back(c->h_tex_table[k]);
+        HIP_TRY(c, hipMemcpy(n->slots_d.p, n->slots.data(), ns * sizeof(NmSlot), hipMemcpyHostToDevice), "upload");
+        HIP_TRY(c, hipMemcpy(n->maps_d.p, maps.data(), maps.size() * sizeof(TexGPU), hipMemcpyHostToDevice), "upload");
+    }
     if (nm) {
         HIP_TRY(c, hipMemcpy(n->slot_of_d.p, n->slot_of.data(), nm * 4, hipMemcpyHostToDevice), "upload");
         HIP_TRY(c, hipMemcpy(n->active_d.p, n->active.data(), nm * 4, hipMemcpyHostToDevice), "upload");
@@ -264,6 +272,7 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     HIP_TRY(c, hipMemcpy(n->block_base_d.p, n->block_base.data(), (ns + 1) * 4, hipMemcpyHostToDevice), "upload");
     const std::vector<float> p = initial_mlp(cfg->init, cfg->seed);
     HIP_TRY(c, hipMemcpy(n->mlp.p, p.data(), kNmParamsPad * 4, hipMemcpyHostToDevice), "upload");
+    HIP_TRY(c, hipMemsetAsync(n->tables.p, 0, kNmStepTables * 64 * 4, s), "clear");
     HIP_TRY(c, hipMemsetAsync(n->mlp_m.p, 0, kNmParamsPad * 4, s), "clear");
     HIP_TRY(c, hipMemsetAsync(n->mlp_v.p, 0, kNmParamsPad * 4, s), "clear");
     HIP_TRY(c, hipMemsetAsync(n->lat_m.p, 0, lat_bytes, s), "clear");
@@ -298,13 +307,13 @@ rsy_result rsy_neural_train(rsy_ctx* c, uint32_t n_steps, float* loss_history) {
     T.loss_base = n->steps;
     T.loss_cap = n_steps;
     hipStream_t s = c->stream;
+    HIP_TRY(c, launch_nm_tables(T, s), "weight tables");
     // a graph of up to 64 consecutive steps (the step counter lives on the device), replayed
     const uint32_t chunk = std::min<uint32_t>(n_steps, 64);
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     HIP_TRY(c, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
-    hipError_t e = hipSuccess;
-    for (uint32_t i = 0; i < chunk && e == hipSuccess; ++i) e = launch_nm_step(T, false, s);
+    hipError_t e = launch_nm_steps(T, chunk, s);
     hipError_t e2 = hipStreamEndCapture(s, &graph);
     if (e != hipSuccess || e2 != hipSuccess) {
         if (graph) (void)hipGraphDestroy(graph);
@@ -316,7 +325,7 @@ rsy_result rsy_neural_train(rsy_ctx* c, uint32_t n_steps, float* loss_history) {
     HIP_TRY(c, hipEventRecord(n->ev0, s), "event");
     uint32_t done = 0;
     for (; done + chunk <= n_steps && e == hipSuccess; done += chunk) e = hipGraphLaunch(exec, s);
-    for (; done < n_steps && e == hipSuccess; ++done) e = launch_nm_step(T, false, s);
+    if (done < n_steps && e == hipSuccess) e = launch_nm_steps(T, n_steps - done, s);
     if (e == hipSuccess) e = hipEventRecord(n->ev1, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     (void)hipGraphExecDestroy(exec);
@@ -487,7 +496,8 @@ rsy_result rsy_neural_gradients(rsy_ctx* c, const uint32_t* material, const floa
     T.ex_offsets = n->tmp[2].as<uint32_t>();
     T.ex_grad_lat = n->tmp[3].as<float>();
     T.ex_grad_mlp = n->tmp[4].as<float>();
-    HIP_TRY(c, launch_nm_step(T, true, s), "gradient kernels");
+    HIP_TRY(c, launch_nm_tables(T, s), "weight tables");
+    HIP_TRY(c, launch_nm_gradient(T, s), "gradient kernels");
     HIP_TRY(c, hipStreamSynchronize(s), "synchronize");
     std::vector<float> g(kNmParamsPad);
     HIP_TRY(c, hipMemcpy(g.data(), n->tmp[4].p, kNmParamsPad * 4, hipMemcpyDeviceToHost), "read gradients");

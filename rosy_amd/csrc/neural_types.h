@@ -17,6 +17,9 @@ constexpr int kNmB2 = kNmW2 + kNmOut * kNmHidden;  // 576
 constexpr int kNmParams = kNmB2 + kNmOut;          // 583
 constexpr int kNmParamsPad = 584;                  // index 583 carries a loss sum where gradients are reduced
 
+// Registers of the training step's weight tables, 64 words each
+constexpr int kNmStepTables = 19;
+
 // Bytes of the MFMA-operand form of the MLP: the FP16 A operands of both layers (3 x 64 entries of
 // 16 bytes), the same as E4M3 codes (3 x 64 entries of 8 bytes), FP32 b2, two FP32 layer scales,
 // the weight-form flag and padding.
