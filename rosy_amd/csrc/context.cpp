@@ -350,6 +350,26 @@ void bind_outputs(Layout& L, const FrameMem& m) {
     }
 }
 
+// Byte offsets of a frame's constants in their device block: view records, shading views, cascades,
+// blend views, scene data.
+struct ConstTables {
+    size_t views, shade_views, shade_cascades, blend_views, scene, bytes;
+};
+ConstTables const_tables(const Layout& L) {
+    ConstTables t{};
+    const auto take = [&](size_t bytes) {
+        const size_t o = t.bytes;
+        t.bytes += (bytes + 255) & ~size_t(255);
+        return o;
+    };
+    t.views = take(L.vg.size() * sizeof(ViewGPU));
+    t.shade_views = take(L.n_camera * sizeof(ShadeView));
+    t.shade_cascades = take(L.n_shadow * sizeof(ShadeCascade));
+    t.blend_views = take(L.n_blend * sizeof(ShadeView));
+    t.scene = take(sizeof(rsy_scene_data));
+    return t;
+}
+
 // Computes the frame's layout and (re)allocates the context's frame buffers for it.
 rsy_result build_layout(rsy_ctx* c, const std::vector<FrameViewDesc>& views, uint32_t tile, uint32_t shade) {
     Layout& L = c->layout;
@@ -367,7 +387,6 @@ rsy_result build_layout(rsy_ctx* c, const std::vector<FrameViewDesc>& views, uin
     if (r != RSY_OK) return r;
     // buffers
     const size_t nv = L.vg.size();
-    HIP_TRY(c, c->views_d.ensure(nv * sizeof(ViewGPU)), "allocate views");
     HIP_TRY(c, c->xv.ensure(size_t(std::max<uint64_t>(1, L.total_xv)) * sizeof(float4)), "allocate vertices");
     HIP_TRY(c, c->recs.ensure(size_t(std::max<uint32_t>(1, L.rec_total)) * sizeof(TriRec)), "allocate records");
     HIP_TRY(c, c->clipq.ensure(size_t(std::max<uint32_t>(1, L.clip_total)) * sizeof(ClipEntry)), "allocate clip queue");
@@ -441,7 +460,6 @@ rsy_result build_layout(rsy_ctx* c, const std::vector<FrameViewDesc>& views, uin
         c->frag_cap = uint32_t(want);
     }
     HIP_TRY(c, c->readback_counters.ensure(nv * kCtrPerView * 4 + 64), "allocate readback");
-    m.views = c->views_d.as<ViewGPU>();
     m.xv = c->xv.as<float4>();
     m.recs = c->recs.as<TriRec>();
     m.bin_tiles = c->bin_tiles.as<uint32_t>();
@@ -466,25 +484,27 @@ rsy_result build_layout(rsy_ctx* c, const std::vector<FrameViewDesc>& views, uin
     m.frag_color = c->frag_color.as<float4>();
     m.frag_mask = c->frag_mask.as<uint8_t>();
     m.frag_cap = c->frag_cap;
-    const size_t nsv = L.n_camera, nsc = L.n_shadow, nbv = L.n_blend;
-    HIP_TRY(c, c->shade_views_d.ensure(std::max<size_t>(1, nsv) * sizeof(ShadeView) + 64), "allocate shade views");
-    HIP_TRY(c, c->shade_cascades_d.ensure(std::max<size_t>(1, nsc) * sizeof(ShadeCascade) + 64), "allocate cascades");
-    HIP_TRY(c, c->blend_shade_views_d.ensure(std::max<size_t>(1, nbv) * sizeof(ShadeView) + 64), "allocate blend views");
-    const size_t staging = ((nv * sizeof(ViewGPU) + 255) & ~size_t(255)) + ((nsv * sizeof(ShadeView) + 255) & ~size_t(255)) +
-                           ((nsc * sizeof(ShadeCascade) + 255) & ~size_t(255)) + nbv * sizeof(ShadeView) + 256;
-    HIP_TRY(c, c->staging.ensure(staging), "allocate staging");
-    m.shade_views = c->shade_views_d.as<ShadeView>();
-    m.shade_cascades = c->shade_cascades_d.as<ShadeCascade>();
-    m.blend_views = c->blend_shade_views_d.as<ShadeView>();
+    m.report = static_cast<uint32_t*>(c->readback_counters.p);
+    // the frame's constants, one after another in one device block and its pinned image
+    const ConstTables at = const_tables(L);
+    HIP_TRY(c, c->consts_d.ensure(at.bytes), "allocate frame constants");
+    HIP_TRY(c, c->staging.ensure(at.bytes), "allocate staging");
+    uint8_t* const k = c->consts_d.as<uint8_t>();
+    m.views = reinterpret_cast<ViewGPU*>(k + at.views);
+    m.shade_views = reinterpret_cast<ShadeView*>(k + at.shade_views);
+    m.shade_cascades = reinterpret_cast<ShadeCascade*>(k + at.shade_cascades);
+    m.blend_views = reinterpret_cast<ShadeView*>(k + at.blend_views);
+    m.scene = k + at.scene;
     bind_outputs(L, m);
     L.valid = true;
     return RSY_OK;
 }
 
-// Per-frame constants (view records, shading views and cascades) go to the device with async copies
-// on the context stream: through `staging` (pinned, at least the tables' size) when given, else
-// straight from host memory.  They are not part of the captured frame graph: a replayed graph reads
-// whatever the last upload left in device memory.
+// Per-frame constants (view records, shading views, cascades, scene data) go to the device with async copies
+// on the context stream: through `staging` (pinned, laid out as their device block) in one copy when given
+// -- a small copy is a blit kernel of 3 us and a gap before the next, and the tables took four with the
+// scene data's -- else table by table straight from host memory.  They are not part of the captured frame
+// graph: a replayed graph reads whatever the last upload left in device memory.
 rsy_result upload_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, void* staging, uint32_t debug_flags) {
     hipStream_t s = c->stream;
     const uint32_t nv = uint32_t(L.vg.size());
@@ -541,28 +561,28 @@ rsy_result upload_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, void* st
         const void* src;
         size_t bytes;
     };
-    const Table tables[4] = {{m.views, L.vg.data(), nv * sizeof(ViewGPU)},
+    const Table tables[5] = {{m.views, L.vg.data(), nv * sizeof(ViewGPU)},
                              {m.shade_views, c->h_shade_views.data(), nsv * sizeof(ShadeView)},
                              {m.shade_cascades, c->h_shade_cascades.data(), nsc * sizeof(ShadeCascade)},
-                             {m.blend_views, c->h_blend_views.data(), nbv * sizeof(ShadeView)}};
-    size_t at = 0;
-    for (const Table& t : tables) {
-        if (!t.bytes) continue;
-        const void* src = t.src;
-        if (staging) {
-            uint8_t* st = static_cast<uint8_t*>(staging) + at;
-            std::memcpy(st, t.src, t.bytes);
-            src = st;
-            at += (t.bytes + 255) & ~size_t(255);
-        }
-        HIP_TRY(c, hipMemcpyAsync(t.dst, src, t.bytes, hipMemcpyHostToDevice, s), "upload frame constants");
+                             {m.blend_views, c->h_blend_views.data(), nbv * sizeof(ShadeView)},
+                             {m.scene, &c->sd, sizeof(c->sd)}};
+    if (staging) {
+        const ConstTables at = const_tables(L);
+        const size_t offsets[5] = {at.views, at.shade_views, at.shade_cascades, at.blend_views, at.scene};
+        for (int k = 0; k < 5; ++k)
+            if (tables[k].bytes) std::memcpy(static_cast<uint8_t*>(staging) + offsets[k], tables[k].src, tables[k].bytes);
+        HIP_TRY(c, hipMemcpyAsync(m.views, staging, at.bytes, hipMemcpyHostToDevice, s), "upload frame constants");
+        return RSY_OK;
     }
+    for (const Table& k : tables)
+        if (k.bytes) HIP_TRY(c, hipMemcpyAsync(k.dst, k.src, k.bytes, hipMemcpyHostToDevice, s), "upload frame constants");
     return RSY_OK;
 }
 
 // Enqueues the kernels of one frame on the context stream (graph-capturable: kernels only).  With
 // `bookkeeping` (the ordinary frame, not while capturing): HIP events around the frame and, with
-// RSY_DEBUG_STAGE_TIMING, between its stages, and the counters copied to the pinned readback buffer.
+// RSY_DEBUG_STAGE_TIMING, between its stages.  m.report (nullable): the last kernel that runs after the
+// counters are final stores them there (pinned host memory).
 rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool capturing, bool bookkeeping) {
     hipStream_t s = c->stream;
     const uint32_t nv = uint32_t(L.vg.size());
@@ -660,6 +680,8 @@ rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool ca
     r.totals = b.totals;
     r.samples = msaa_of(c);
     r.grid = b.raster_grid;
+    r.counters = m.counters;
+    if (!L.n_blend) r.report = m.report;
     HIP_TRY(c, launch_raster(r, s), "raster kernel");
     if (timing) HIP_TRY(c, hipEventRecord(c->ev_stage[2], s), "event");
 
@@ -671,7 +693,7 @@ rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool ca
         sh.cascades = m.shade_cascades;
         sh.n_cascades = uint32_t(c->h_shade_cascades.size());
         sh.pcf_mode = c->rs.pcf_mode;
-        sh.scene = c->scene_d.p;
+        sh.scene = m.scene;
         sh.draws = c->lists_d[1].as<DrawGPU>();
         sh.n_draws = uint32_t(c->lists[1].size());
         sh.indices = g.indices;
@@ -712,6 +734,8 @@ rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool ca
             bl.frag_mask = m.frag_mask;
             bl.frag_cap = m.frag_cap;
             bl.samples = msaa_of(c);
+            bl.totals = m.totals;
+            bl.report = m.report;
             sb.views = m.blend_views;
             sb.n_views = uint32_t(c->h_blend_views.size());
             sb.draws = c->lists_d[2].as<DrawGPU>();
@@ -742,10 +766,6 @@ rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool ca
     }
     if (timing) HIP_TRY(c, hipEventRecord(c->ev_stage[4], s), "event");
     if (events) {
-        HIP_TRY(c, hipMemcpyAsync(c->readback_counters.p, m.counters, nv * kCtrPerView * 4, hipMemcpyDeviceToHost, s),
-                "readback");
-        HIP_TRY(c, hipMemcpyAsync(static_cast<uint8_t*>(c->readback_counters.p) + nv * kCtrPerView * 4, m.totals, 16,
-                                  hipMemcpyDeviceToHost, s), "readback");
         HIP_TRY(c, hipEventRecord(c->ev_end, s), "event");
     }
     return RSY_OK;
@@ -1193,10 +1213,7 @@ rsy_result rsy_update(rsy_ctx* c, const rsy_scene_data* sd, const rsy_raster_sta
         c->rs = *state;
         if (raster_changed) c->layout.valid = false;
     }
-    HIP_TRY(c, hipSetDevice(c->device), "set device");
-    HIP_TRY(c, hipStreamSynchronize(c->stream), "synchronize");
-    c->sd = *sd;
-    HIP_TRY(c, hipMemcpy(c->scene_d.p, sd, sizeof(rsy_scene_data), hipMemcpyHostToDevice), "upload scene data");
+    c->sd = *sd;  // uploaded with every frame's constants
     c->has_scene = true;
     return RSY_OK;
 }
@@ -1249,10 +1266,6 @@ rsy_result rsy_render_graph(rsy_ctx* c, const rsy_frame_desc* frame, uint32_t n_
     }
     HIP_TRY(c, hipEventRecord(c->ev_begin, c->stream), "event");
     for (uint32_t i = 0; i < n_replays; ++i) HIP_TRY(c, hipGraphLaunch(c->graph_exec, c->stream), "graph launch");
-    const uint32_t nv = uint32_t(c->layout.vg.size());
-    HIP_TRY(c, hipMemcpyAsync(c->readback_counters.p, c->counters.p, nv * kCtrPerView * 4, hipMemcpyDeviceToHost, c->stream), "readback");
-    HIP_TRY(c, hipMemcpyAsync(static_cast<uint8_t*>(c->readback_counters.p) + nv * kCtrPerView * 4, c->totals.p, 16,
-                              hipMemcpyDeviceToHost, c->stream), "readback");
     HIP_TRY(c, hipEventRecord(c->ev_end, c->stream), "event");
     HIP_TRY(c, hipStreamSynchronize(c->stream), "synchronize");
     const bool over = collect_stats(c);
@@ -1310,6 +1323,7 @@ rsy_result rsy_render_noalloc(rsy_ctx* c, const rsy_frame_desc* frame, const rsy
     m.totals = reinterpret_cast<uint32_t*>(take(32));
     m.shade_views = reinterpret_cast<ShadeView*>(take(L.n_camera * sizeof(ShadeView)));
     m.shade_cascades = reinterpret_cast<ShadeCascade*>(take(L.n_shadow * sizeof(ShadeCascade)));
+    m.scene = c->scene_d.p;
     m.vblocks = reinterpret_cast<BlockEntry*>(take(L.vblocks.size() * sizeof(BlockEntry)));
     m.tblocks = reinterpret_cast<BlockEntry*>(take(L.tblocks.size() * sizeof(BlockEntry)));
     m.block_valid = reinterpret_cast<uint32_t*>(take(L.tblocks.size() * 4));

@@ -156,6 +156,8 @@ struct FrameMem {
     ShadeView* shade_views = nullptr;
     ShadeCascade* shade_cascades = nullptr;
     ShadeView* blend_views = nullptr;
+    void* scene = nullptr;         // rsy_scene_data
+    uint32_t* report = nullptr;    // host: the counters and totals of the frame (null: not wanted)
     // the blended pass's fragments
     uint4* frags = nullptr;
     uint32_t* frag_keys = nullptr;
@@ -227,15 +229,15 @@ struct rsy_ctx {
     rsy_scene_data sd{};
     rsy_raster_state rs{};
     bool has_scene = false;
-    rsy::DevBuf scene_d;
+    rsy::DevBuf scene_d;  // of the allocation-free frame (the ordinary frame's is among its constants)
 
     // frame buffers
     rsy::Layout layout;
     rsy::FrameMem mem;            // the ordinary frame's addresses (into the buffers below)
     rsy::Layout static_layout;    // the allocation-free frame's layout (host tables only)
     std::vector<rsy::FrameViewDesc> static_views;
-    rsy::DevBuf views_d, xv, recs, bin_tiles, shade_recs, clipq, counters, bin_counts, bin_offsets, pair_slots, big_pairs, block_valid, totals,
-        lists_mem, vblocks_d, tblocks_d, shade_views_d, shade_cascades_d, items,
+    rsy::DevBuf consts_d, xv, recs, bin_tiles, shade_recs, clipq, counters, bin_counts, bin_offsets, pair_slots, big_pairs, block_valid, totals,
+        lists_mem, vblocks_d, tblocks_d, items,
         draw_culled, scan_partial;
     uint32_t list_cap = 0;
     uint32_t rec_scale = 1;  // grows on overflow
@@ -244,7 +246,6 @@ struct rsy_ctx {
     rsy::DevBuf frags, frag_keys, frag_color, frag_mask;  // the blended pass's fragments
     std::vector<rsy::DevBuf> sample_color;  // per camera view, 4 samples with a blended pass: colour planes
     uint32_t frag_cap = 0;
-    rsy::DevBuf blend_shade_views_d;
     std::vector<rsy::ShadeView> h_blend_views;
     rsy::PinnedBuf staging, readback_counters;
     std::vector<rsy::ShadeView> h_shade_views;

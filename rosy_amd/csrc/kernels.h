@@ -101,6 +101,8 @@ struct RasterLaunch {
     const uint32_t* totals;  // [3] work items
     uint32_t samples;  // of the camera views (1 or 4)
     uint32_t grid;     // workgroups: one per work item (the last frame's count, with slack)
+    const uint32_t* counters;  // per view
+    uint32_t* report;  // nullable: host memory for every view's counters, then totals[0..3]
 };
 
 // The blended pass over the bins of the blend views (one launch).
@@ -123,6 +125,8 @@ struct BlendLaunch {
     uint8_t* frag_mask;     // 4 samples: per fragment, the samples it covers and passes the depth test at
     uint32_t frag_cap;
     uint32_t samples;       // samples per pixel of the camera views (1 or 4)
+    const uint32_t* totals;
+    uint32_t* report;       // nullable: as RasterLaunch::report
 };
 
 // Per-pixel shading inputs of one camera view.

@@ -1025,7 +1025,8 @@ __global__ __launch_bounds__(256) void k_scatter(const ViewGPU* views, const uin
 template <int T, int N>
 __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n_views, const uint32_t* lists,
                                                 uint32_t list_cap, const TriRec* recs, uint64_t rec_cap_total,
-                                                const uint4* items, const uint32_t* totals) {
+                                                const uint4* items, const uint32_t* totals, const uint32_t* counters,
+                                                uint32_t* report) {
     constexpr int S = T + 1;  // padded row stride (words)
     __shared__ unsigned long long tile[N * T * S];  // camera views: one plane per sample
     __shared__ TriRec chunk_recs[kChunkRecs];
@@ -1039,6 +1040,8 @@ __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n
     // beside the count (blockIdx.x < gridDim.x <= the table's capacity).
     const uint32_t n_items = totals[3];
     const uint4 it = items[blockIdx.x];
+    // the last workgroup (past the items, as a rule) also reports the frame's counters
+    if (report && blockIdx.x + 1u == gridDim.x) report_counters(report, counters, n_views, totals);
     // (the test reads the item too, which keeps its load beside the count's instead of after the
     // branch; an item's record count never reaches 2^31)
     if (blockIdx.x >= n_items || int32_t(it.z) < 0) return;
@@ -1168,7 +1171,7 @@ hipError_t launch_raster(const RasterLaunch& r, hipStream_t s) {
     if (grid == 0) return hipSuccess;
 #define RSY_RASTER(T, N)                                                                                         \
     hipLaunchKernelGGL((k_raster<T, N>), dim3(grid), dim3(256), 0, s, r.views, r.n_views, r.lists, r.list_cap, \
-                       r.recs, r.rec_cap_total, r.items, r.totals)
+                       r.recs, r.rec_cap_total, r.items, r.totals, r.counters, r.report)
     if (r.samples == 1) {
         if (r.tile == 8) RSY_RASTER(8, 1);
         else if (r.tile == 16) RSY_RASTER(16, 1);

@@ -906,6 +906,7 @@ __device__ inline float4 blend_over(float4 dst, float4 f) {
 
 template <int T, int N>
 __global__ __launch_bounds__(256) void k_blend_resolve(const BlendLaunch B, const ShadeLaunch L) {
+    if (B.report && blockIdx.x + 1u == gridDim.x) report_counters(B.report, B.counters, B.n_views, B.totals);
     uint32_t vi = 0;
     while (vi + 1 < L.n_views && L.views[vi + 1].block_base <= blockIdx.x) ++vi;
     const ShadeView& SV = L.views[vi];
