@@ -1077,40 +1077,58 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     if (n_materials) HIP_TRY(c, hipMemcpy(c->materials.p, materials, n_materials * sizeof(rsy_gpu_material), hipMemcpyHostToDevice), "upload materials");
     if (n_textures) HIP_TRY(c, hipMemcpy(c->tex_table.p, table.data(), n_textures * sizeof(TexGPU), hipMemcpyHostToDevice), "upload textures");
     if (staging) HIP_TRY(c, c->tex_staging.ensure(staging), "allocate texture staging");
+    // the given levels first (a BC7 image is decoded while the next image is copied), then every built chain and
+    // the alpha test of every image, in a few launches over all of them
+    std::vector<MipJob> jobs;  // [0, n_textures): every image; then the ones whose chains are built
+    uint32_t max_w = 0, max_h = 0, max_levels = 0;
+    for (uint32_t t = 0; t < n_textures; ++t) jobs.push_back({table[t].offset, table[t].width, table[t].height, table[t].channels, table[t].srgb, table[t].levels, 0u});
+    for (uint32_t t = 0; t < n_textures; ++t)
+        if (textures[t].mip_levels == RSY_MIPS_BUILD && table[t].levels > 1) {
+            jobs.push_back(jobs[t]);
+            max_w = std::max(max_w, table[t].width);
+            max_h = std::max(max_h, table[t].height);
+            max_levels = std::max(max_levels, table[t].levels);
+        }
+    if (n_textures) {
+        HIP_TRY(c, c->tex_jobs.ensure(jobs.size() * sizeof(MipJob)), "allocate texture jobs");
+        HIP_TRY(c, c->tex_flags.ensure(size_t(n_textures) * 4), "allocate texture flags");
+        HIP_TRY(c, hipMemcpyAsync(c->tex_jobs.p, jobs.data(), jobs.size() * sizeof(MipJob), hipMemcpyHostToDevice, c->stream),
+                "upload texture jobs");
+        if (max_levels && !c->mip_tables.p) {
+            HIP_TRY(c, c->mip_tables.ensure(512 * sizeof(double)), "allocate mip tables");
+            HIP_TRY(c, launch_mip_tables(c->mip_tables.as<double>(), c->stream), "mip tables");
+        }
+    }
     uint64_t staged = 0;  // every BC7 image's blocks go to their own part of the staging buffer
     for (uint32_t t = 0; t < n_textures; ++t) {
-        // the given levels (BC7 decoded on the GPU), then the built ones, each from the one above
         const rsy_texture_desc& d = textures[t];
         const TexGPU& g = table[t];
         const bool bc7 = d.format == RSY_TEX_BC7_SRGB || d.format == RSY_TEX_BC7_UNORM;
         const uint32_t given = d.mip_levels == RSY_MIPS_BUILD ? 1u : std::max(1u, d.mip_levels);
-        const uint8_t* src = static_cast<const uint8_t*>(d.pixels);
         uint8_t* base = c->texels.as<uint8_t>() + g.offset;
         if (bc7) {
             uint64_t n = 0;
             for (uint32_t l = 0; l < given; ++l)
                 n += uint64_t((mip_extent(g.width, l) + 3) / 4) * ((mip_extent(g.height, l) + 3) / 4) * 16;
-            HIP_TRY(c, hipMemcpyAsync(c->tex_staging.as<uint8_t>() + staged, src, n, hipMemcpyHostToDevice, c->stream),
-                    "upload BC7 blocks");
+            uint8_t* blocks = c->tex_staging.as<uint8_t>() + staged;
+            HIP_TRY(c, hipMemcpyAsync(blocks, d.pixels, n, hipMemcpyHostToDevice, c->stream), "upload BC7 blocks");
+            HIP_TRY(c, launch_bc7_decode(blocks, g.width, g.height, given, reinterpret_cast<uint32_t*>(base), c->stream),
+                    "BC7 decode");
+            staged += n;
+        } else {  // the levels follow one another on both sides
+            HIP_TRY(c, hipMemcpyAsync(base, d.pixels, mip_offset(g.width, g.height, g.channels, given), hipMemcpyHostToDevice,
+                                      c->stream), "upload texels");
         }
-        for (uint32_t l = 0; l < given; ++l) {
-            const uint32_t w = mip_extent(g.width, l), h = mip_extent(g.height, l);
-            uint8_t* dst = base + mip_offset(g.width, g.height, g.channels, l);
-            if (bc7) {
-                const uint64_t n = uint64_t((w + 3) / 4) * ((h + 3) / 4) * 16;
-                HIP_TRY(c, launch_bc7_decode(c->tex_staging.as<uint8_t>() + staged, w, h, reinterpret_cast<uint32_t*>(dst),
-                                             c->stream), "BC7 decode");
-                staged += n;
-            } else {
-                const uint64_t n = uint64_t(w) * h * g.channels;
-                HIP_TRY(c, hipMemcpy(dst, src, n, hipMemcpyHostToDevice), "upload texels");
-                src += n;
-            }
-        }
-        for (uint32_t l = given; l < g.levels; ++l)
-            HIP_TRY(c, launch_build_mip(base + mip_offset(g.width, g.height, g.channels, l - 1), mip_extent(g.width, l - 1),
-                                        mip_extent(g.height, l - 1), base + mip_offset(g.width, g.height, g.channels, l),
-                                        g.channels, g.srgb, c->stream), "build mip level");
+    }
+    std::vector<uint32_t> opaque(n_textures);
+    if (n_textures) {
+        const MipJob* dj = c->tex_jobs.as<MipJob>();
+        if (max_levels)
+            HIP_TRY(c, launch_build_mips(dj + n_textures, uint32_t(jobs.size() - n_textures), max_w, max_h, max_levels,
+                                         c->texels.as<uint8_t>(), c->mip_tables.as<double>(), c->stream), "build mip levels");
+        HIP_TRY(c, launch_alpha_test(dj, n_textures, c->texels.as<uint8_t>(), c->tex_flags.as<uint32_t>(), c->stream), "alpha test");
+        HIP_TRY(c, hipMemcpyAsync(opaque.data(), c->tex_flags.p, size_t(n_textures) * 4, hipMemcpyDeviceToHost, c->stream),
+                "read alpha test");
     }
     HIP_TRY(c, hipStreamSynchronize(c->stream), "synchronize");
     if (n_samplers) HIP_TRY(c, hipMemcpy(c->samplers.p, samplers, n_samplers * sizeof(rsy_sampler), hipMemcpyHostToDevice), "upload samplers");
@@ -1133,21 +1151,9 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
         }
     c->tex_opaque.assign(n_textures, 0);
     c->any_mips = false;
-    std::vector<uint8_t> decoded;
     for (uint32_t t = 0; t < n_textures; ++t) {
         c->any_mips |= table[t].levels > 1;
-        if (table[t].channels != 4) continue;
-        const uint64_t n = uint64_t(table[t].width) * table[t].height;
-        const uint8_t* px = static_cast<const uint8_t*>(textures[t].pixels);
-        if (textures[t].format == RSY_TEX_BC7_SRGB || textures[t].format == RSY_TEX_BC7_UNORM) {
-            decoded.resize(n * 4);  // level 0 as decoded
-            HIP_TRY(c, hipMemcpy(decoded.data(), c->texels.as<uint8_t>() + table[t].offset, n * 4, hipMemcpyDeviceToHost),
-                    "read decoded texels");
-            px = decoded.data();
-        }
-        bool opaque = true;
-        for (uint64_t i = 0; i < n && opaque; ++i) opaque = px[4 * i + 3] == 255;
-        c->tex_opaque[t] = opaque ? 1 : 0;
+        if (table[t].channels == 4) c->tex_opaque[t] = opaque[t] ? 1 : 0;
     }
     // a decoder trained on the previous materials no longer applies
     destroy_neural(c->neural);

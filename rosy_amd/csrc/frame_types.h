@@ -147,6 +147,15 @@ __host__ __device__ inline uint64_t mip_offset(uint32_t w, uint32_t h, uint32_t 
     return o;
 }
 
+// One image of the upload kernels (mip chains, alpha test).
+struct MipJob {
+    uint64_t offset;  // bytes into the texel pool
+    uint32_t width, height;
+    uint32_t channels, srgb;
+    uint32_t levels;
+    uint32_t pad;
+};
+
 // The standard locations of a 4-sample pixel, (0.375, 0.125), (0.875, 0.375), (0.125, 0.625) and
 // (0.625, 0.875), in 1/256 pixel.
 __host__ __device__ constexpr int32_t msaa_x(int s) { return s == 0 ? 96 : s == 1 ? 224 : s == 2 ? 32 : 160; }

@@ -266,10 +266,14 @@ struct NmPointLaunch {
     float* out;  // [n][7]
 };
 
-// texture upload: BC7 blocks of a width x height image into RGBA8 texels; mip level l + 1 from level l
-hipError_t launch_bc7_decode(const void* blocks, uint32_t width, uint32_t height, uint32_t* rgba, hipStream_t s);
-hipError_t launch_build_mip(const uint8_t* src, uint32_t src_w, uint32_t src_h, uint8_t* dst, uint32_t channels,
-                            uint32_t srgb, hipStream_t s);
+// texture upload: the BC7 blocks of an image's levels into RGBA8 texels; the byte tables of the mip filter; the
+// chains of the images in `jobs`, each from its level 0; flags[i] = 1 when image i is opaque (four channels)
+hipError_t launch_bc7_decode(const void* blocks, uint32_t width, uint32_t height, uint32_t levels, uint32_t* rgba,
+                             hipStream_t s);
+hipError_t launch_mip_tables(double* tables, hipStream_t s);
+hipError_t launch_build_mips(const MipJob* jobs, uint32_t n_jobs, uint32_t max_width, uint32_t max_height,
+                             uint32_t max_levels, uint8_t* texels, const double* tables, hipStream_t s);
+hipError_t launch_alpha_test(const MipJob* jobs, uint32_t n_jobs, const uint8_t* texels, uint32_t* flags, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 hipError_t launch_geometry(const GeometryLaunch& g, hipStream_t s);
 hipError_t launch_binning(const BinLaunch& b, hipStream_t s);
