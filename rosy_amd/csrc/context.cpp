@@ -8,9 +8,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <new>
 #include <string>
 #include <vector>
@@ -704,6 +706,8 @@ rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool ca
         sh.textures = c->tex_table.as<TexGPU>();
         sh.n_textures = c->n_textures;
         sh.texels = c->texels.as<uint8_t>();
+        sh.packs = c->packs.as<PackGPU>();
+        sh.packed = c->packed.as<uint8_t>();
         sh.samplers = c->samplers.p;
         sh.n_samplers = c->n_samplers;
         std::memcpy(sh.clear_color, c->rs.clear_color, sizeof(sh.clear_color));
@@ -1036,6 +1040,56 @@ rsy_result rsy_set_geometry(rsy_ctx* c, const rsy_position* vertices, uint64_t n
     return RSY_OK;
 }
 
+namespace {
+// The materials that can be sampled as one packed image: a four-channel sRGB albedo, a two-channel linear normal
+// map and a metallic-roughness map (mixmap when present) of the same size and level count, sampled bilinearly
+// with the same addressing.  Others (a map missing, a four-channel normal map, sizes that differ, nearest filtering)
+// keep their maps, at the cost they had: one packed sample needs one set of coordinates.  Materials
+// with the same maps share one image.  Returns the bytes of the packed texels.
+uint64_t plan_packs(const rsy_gpu_material* materials, uint32_t n_materials, const std::vector<TexGPU>& table,
+                    const rsy_sampler* samplers, uint32_t n_samplers, std::vector<PackGPU>& packs,
+                    std::vector<PackJob>& jobs, uint32_t& max_tiles) {
+    packs.assign(n_materials, PackGPU{});
+    std::map<std::array<uint32_t, 3>, uint64_t> made;  // maps -> offset
+    uint64_t bytes = 0;
+    auto sampler_mode = [&](uint32_t i) {
+        if (i >= n_samplers) return 2u << kPackWrapS | 2u << kPackWrapT;
+        const rsy_sampler& s = samplers[i];
+        const uint32_t ws = std::min<uint32_t>(s.wrap_s, 2u), wt = std::min<uint32_t>(s.wrap_t, 2u);  // 0 clamps, 1 mirrors, others repeat
+        if (s.mag_filter <= 2 || s.min_filter <= 2) return ~0u;  // nearest: not packed
+        return ws << kPackWrapS | wt << kPackWrapT;
+    };
+    for (uint32_t m = 0; m < n_materials; ++m) {
+        const rsy_gpu_material& g = materials[m];
+        const bool use_mix = g.mixmap_sampled_image_index < table.size();
+        const uint32_t ci = g.color_sampled_image_index, ni = g.normal_sampled_image_index;
+        const uint32_t mi = use_mix ? g.mixmap_sampled_image_index : g.metallic_sampled_image_index;
+        if (ci >= table.size() || ni >= table.size() || mi >= table.size()) continue;
+        const TexGPU &c = table[ci], &n = table[ni], &r = table[mi];
+        if (c.channels != 4 || !c.srgb || n.channels != 2 || n.srgb) continue;
+        auto alike = [&](const TexGPU& t) { return t.width == c.width && t.height == c.height && t.levels == c.levels; };
+        if (!alike(n) || !alike(r)) continue;
+        const uint32_t mode = sampler_mode(g.color_sampler_index);
+        if (mode == ~0u || sampler_mode(g.normal_sampler_index) != mode ||
+            sampler_mode(use_mix ? g.mixmap_sampler_index : g.metallic_sampler_index) != mode)
+            continue;
+        const auto key = std::array<uint32_t, 3>{ci, ni, mi};
+        auto at = made.find(key);
+        if (at == made.end()) {
+            at = made.emplace(key, bytes).first;
+            jobs.push_back({c, n, r, bytes});
+            uint32_t tiles = 0;
+            for (uint32_t l = 0; l < c.levels; ++l) tiles += pack_tiles(c.width, c.height, l);
+            max_tiles = std::max(max_tiles, tiles);
+            bytes += uint64_t(tiles) * 128;
+        }
+        packs[m] = {at->second, c.width, c.height, c.levels,
+                    mode | (r.srgb ? kPackMrSrgb : 0u)};
+    }
+    return bytes;
+}
+}  // namespace
+
 rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint32_t n_materials,
                              const rsy_texture_desc* textures, uint32_t n_textures, const rsy_sampler* samplers,
                              uint32_t n_samplers) {
@@ -1043,6 +1097,7 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     if ((n_materials && !materials) || (n_textures && !textures) || (n_samplers && !samplers))
         return fail(c, RSY_INVALID_ARGUMENT, "null material pointer");
     std::vector<TexGPU> table(n_textures);
+    std::vector<PackGPU> packs;
     uint64_t pool = 0, staging = 0;
     for (uint32_t t = 0; t < n_textures; ++t) {
         const rsy_texture_desc& d = textures[t];
@@ -1129,6 +1184,25 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
         HIP_TRY(c, launch_alpha_test(dj, n_textures, c->texels.as<uint8_t>(), c->tex_flags.as<uint32_t>(), c->stream), "alpha test");
         HIP_TRY(c, hipMemcpyAsync(opaque.data(), c->tex_flags.p, size_t(n_textures) * 4, hipMemcpyDeviceToHost, c->stream),
                 "read alpha test");
+    }
+    std::vector<PackJob> pack_jobs;
+    uint32_t pack_tiles_max = 0;
+    const uint64_t pack_bytes = plan_packs(materials, n_materials, table, samplers, n_samplers, packs, pack_jobs, pack_tiles_max);
+    HIP_TRY(c, c->packs.ensure(std::max<size_t>(1, n_materials) * sizeof(PackGPU)), "allocate packed materials");
+    if (c->packed.ensure(std::max<uint64_t>(256, pack_bytes)) != hipSuccess) {
+        hipGetLastError();  // no room for a second copy of the texels: the maps are sampled one by one
+        for (PackGPU& k : packs) k.levels = 0;
+        pack_jobs.clear();
+    }
+    if (n_materials)
+        HIP_TRY(c, hipMemcpyAsync(c->packs.p, packs.data(), packs.size() * sizeof(PackGPU), hipMemcpyHostToDevice, c->stream),
+                "upload packed materials");
+    if (!pack_jobs.empty()) {
+        HIP_TRY(c, c->pack_jobs.ensure(pack_jobs.size() * sizeof(PackJob)), "allocate pack jobs");
+        HIP_TRY(c, hipMemcpyAsync(c->pack_jobs.p, pack_jobs.data(), pack_jobs.size() * sizeof(PackJob), hipMemcpyHostToDevice,
+                                  c->stream), "upload pack jobs");
+        HIP_TRY(c, launch_pack(c->pack_jobs.as<PackJob>(), uint32_t(pack_jobs.size()), pack_tiles_max, c->texels.as<uint8_t>(),
+                               c->packed.as<uint8_t>(), c->stream), "pack materials");
     }
     HIP_TRY(c, hipStreamSynchronize(c->stream), "synchronize");
     if (n_samplers) HIP_TRY(c, hipMemcpy(c->samplers.p, samplers, n_samplers * sizeof(rsy_sampler), hipMemcpyHostToDevice), "upload samplers");

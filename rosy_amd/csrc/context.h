@@ -217,6 +217,7 @@ struct rsy_ctx {
     std::vector<uint8_t> tex_opaque;  // four-channel texture whose alpha is 255 everywhere
     rsy::DevBuf tex_staging;          // BC7 blocks on their way to the decoder
     rsy::DevBuf tex_jobs, tex_flags;  // the upload kernels' images and alpha-test results
+    rsy::DevBuf packs, packed, pack_jobs;  // packed materials: per material, their texels, the upload's jobs
     rsy::DevBuf mip_tables;           // byte values of the mip filter (made at the first built chain)
     bool any_mips = false;            // some texture has more than one level (LOD sampling)
     // draw lists: 0 = shadow (all), 1 = opaque (!blended), 2 = blended (the blended pass)

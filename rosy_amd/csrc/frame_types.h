@@ -147,6 +147,33 @@ __host__ __device__ inline uint64_t mip_offset(uint32_t w, uint32_t h, uint32_t 
     return o;
 }
 
+// One material's albedo, normal and metallic-roughness maps as a single image of eight-byte texels (sRGB albedo with
+// alpha, linear normal XY, metalness, roughness), for materials whose maps have one size and one bilinear sampler.
+// Texels lie in tiles of 4 x 4, each one 128-byte line, tiles row by row, level after level.
+struct PackGPU {
+    uint64_t offset;  // bytes into the packed texels
+    uint32_t width, height;
+    uint32_t levels;  // 0: not packed, the maps are sampled one by one
+    uint32_t mode;    // kPack* bits
+};
+constexpr uint32_t kPackWrapS = 0, kPackWrapT = 2;  // shifts of the two-bit addressing modes
+constexpr uint32_t kPackMrSrgb = 16;               // metalness and roughness are sRGB-coded
+static_assert(sizeof(PackGPU) == 24, "PackGPU is 24 bytes");
+
+__host__ __device__ inline uint32_t pack_tiles(uint32_t w, uint32_t h, uint32_t l) {
+    return ((mip_extent(w, l) + 3) / 4) * ((mip_extent(h, l) + 3) / 4);
+}
+// Texel index of (x, y) in a level that is `width` texels wide.
+__host__ __device__ inline uint32_t pack_texel(uint32_t width, uint32_t x, uint32_t y) {
+    return ((y >> 2) * ((width + 3) / 4) + (x >> 2)) * 16 + (y & 3u) * 4 + (x & 3u);
+}
+
+// One packed image to be made: its maps and where it goes.
+struct PackJob {
+    TexGPU color, normal, mr;
+    uint64_t offset;
+};
+
 // One image of the upload kernels (mip chains, alpha test).
 struct MipJob {
     uint64_t offset;  // bytes into the texel pool

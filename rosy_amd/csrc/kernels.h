@@ -173,6 +173,8 @@ struct ShadeLaunch {
     const TexGPU* textures;
     uint32_t n_textures;
     const uint8_t* texels;
+    const PackGPU* packs;  // per material
+    const uint8_t* packed;
     const void* samplers;  // rsy_sampler
     uint32_t n_samplers;
     float clear_color[4];
@@ -274,6 +276,9 @@ hipError_t launch_mip_tables(double* tables, hipStream_t s);
 hipError_t launch_build_mips(const MipJob* jobs, uint32_t n_jobs, uint32_t max_width, uint32_t max_height,
                              uint32_t max_levels, uint8_t* texels, const double* tables, hipStream_t s);
 hipError_t launch_alpha_test(const MipJob* jobs, uint32_t n_jobs, const uint8_t* texels, uint32_t* flags, hipStream_t s);
+// the packed images of `jobs` (at most max_tiles tiles each over all of their levels)
+hipError_t launch_pack(const PackJob* jobs, uint32_t n_jobs, uint32_t max_tiles, const uint8_t* texels, uint8_t* packed,
+                       hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 hipError_t launch_geometry(const GeometryLaunch& g, hipStream_t s);
 hipError_t launch_binning(const BinLaunch& b, hipStream_t s);

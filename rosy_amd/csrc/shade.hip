@@ -365,7 +365,7 @@ struct Fragment {
 // decoder's outputs `dec` replace the albedo, normal and metallic-roughness samples of the plain
 // textures.  kUniformDraw: every live lane of the wave shades the same draw.
 template <bool kUniformDraw, bool kLod = false>
-__device__ inline Fragment shade_pixel(const ShadeLaunch& L, const ShadeShared& S, const PixelGeom& pg, bool use_dec,
+__device__ __forceinline__ Fragment shade_pixel(const ShadeLaunch& L, const ShadeShared& S, const PixelGeom& pg, bool use_dec,
                                        const float (&dec)[kNmOut]) {
     using R = std::conditional_t<kUniformDraw, WaveRecords, LaneRecords>;
     const SceneP sd = (SceneP)(L.scene);
@@ -434,34 +434,54 @@ __device__ inline Fragment shade_pixel(const ShadeLaunch& L, const ShadeShared& 
             smetal = dec[5];
             srough = dec[6];
         } else {
-            if (sd->normal_maps_enabled == 1 && valid_index(nti) && nti < L.n_textures) {
-                const TexGPU tg = R::load(textures + nti);
-                const uint32_t si = md->normal_sampler_index;
-                const SamplerState smp = si < L.n_samplers ? sampler_state(R::load(samplers + si)) : SamplerState{};
-                const float4 s = sample(tg, smp);
-                f3 m = mk(s.x * 2.f - 1.f, s.y * 2.f - 1.f, s.z * 2.f - 1.f);
-                if (tg.channels == 2) m.z = __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - m.x * m.x - m.y * m.y));
+            auto bend = [&](f3 m) {
                 const f3 n = normalize(bn);
                 const f3 tt = normalize(btan - n * dot(btan, n));
                 const f3 bb = normalize(cross(bn, btan) * sigma);
                 light_normal = normalize(tt * m.x + bb * m.y + n * m.z);
-            }
-            const uint32_t cti = md->color_sampled_image_index;
-            if (valid_index(cti) && cti < L.n_textures) {
-                const TexGPU tg = R::load(textures + cti);
-                const uint32_t si = md->color_sampler_index;
-                const SamplerState smp = si < L.n_samplers ? sampler_state(R::load(samplers + si)) : SamplerState{};
-                image = sample(tg, smp);
+            };
+            const PackGPU pk = R::load(R::ptr(L.packs) + dr.material);
+            if (pk.levels != 0u) {
+                const uint2* base = reinterpret_cast<const uint2*>(L.packed + pk.offset);
+                PackSample s;
+                if constexpr (kLod) s = sample_pack_lod(base, pk, tu, tv, dudx, dvdx, dudy, dvdy, lut);
+                else s = sample_pack(base, pk, tu, tv, lut);
+                if (sd->normal_maps_enabled == 1) {
+                    f3 m = mk(s.nx * 2.f - 1.f, s.ny * 2.f - 1.f, 0.f);
+                    m.z = __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - m.x * m.x - m.y * m.y));
+                    bend(m);
+                }
+                image = s.color;
                 alpha = fminf(image.w, alpha);
-            }
-            const uint32_t mixti = md->mixmap_sampled_image_index, metti = md->metallic_sampled_image_index;
-            const bool use_mix = valid_index(mixti) && mixti < L.n_textures;
-            const uint32_t mti = use_mix ? mixti : metti;
-            const uint32_t msi = use_mix ? md->mixmap_sampler_index : md->metallic_sampler_index;
-            if (valid_index(mti) && mti < L.n_textures) {
-                const TexGPU tg = R::load(textures + mti);
-                const SamplerState smp = msi < L.n_samplers ? sampler_state(R::load(samplers + msi)) : SamplerState{};
-                mr_from(int(tg.channels), sample(tg, smp), srough, smetal);
+                smetal = s.metal;
+                srough = s.rough;
+            } else {
+                if (sd->normal_maps_enabled == 1 && valid_index(nti) && nti < L.n_textures) {
+                    const TexGPU tg = R::load(textures + nti);
+                    const uint32_t si = md->normal_sampler_index;
+                    const SamplerState smp = si < L.n_samplers ? sampler_state(R::load(samplers + si)) : SamplerState{};
+                    const float4 s = sample(tg, smp);
+                    f3 m = mk(s.x * 2.f - 1.f, s.y * 2.f - 1.f, s.z * 2.f - 1.f);
+                    if (tg.channels == 2) m.z = __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - m.x * m.x - m.y * m.y));
+                    bend(m);
+                }
+                const uint32_t cti = md->color_sampled_image_index;
+                if (valid_index(cti) && cti < L.n_textures) {
+                    const TexGPU tg = R::load(textures + cti);
+                    const uint32_t si = md->color_sampler_index;
+                    const SamplerState smp = si < L.n_samplers ? sampler_state(R::load(samplers + si)) : SamplerState{};
+                    image = sample(tg, smp);
+                    alpha = fminf(image.w, alpha);
+                }
+                const uint32_t mixti = md->mixmap_sampled_image_index, metti = md->metallic_sampled_image_index;
+                const bool use_mix = valid_index(mixti) && mixti < L.n_textures;
+                const uint32_t mti = use_mix ? mixti : metti;
+                const uint32_t msi = use_mix ? md->mixmap_sampler_index : md->metallic_sampler_index;
+                if (valid_index(mti) && mti < L.n_textures) {
+                    const TexGPU tg = R::load(textures + mti);
+                    const SamplerState smp = msi < L.n_samplers ? sampler_state(R::load(samplers + msi)) : SamplerState{};
+                    mr_from(int(tg.channels), sample(tg, smp), srough, smetal);
+                }
             }
         }
     }
