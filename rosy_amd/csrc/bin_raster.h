@@ -64,7 +64,6 @@ __device__ inline void report_counters(uint32_t* report, const uint32_t* counter
 }
 
 constexpr uint32_t kItemRecs = 256;   // records per raster work item (one per thread)
-constexpr uint32_t kChunkRecs = 128;  // records staged in LDS at a time
 
 // Exclusive prefix sum over the workgroup (wave scans by DPP, wave totals through LDS).
 // Every thread of the block must call it; it synchronises the block.  kTailSync = false leaves out
@@ -187,6 +186,15 @@ struct FillFragMS {  // blend view: append key | passing-sample mask << 28 to th
     }
 };
 
+// Edge-value products.  A record that is not wide has every coordinate difference of its edges and of its pixels
+// under 2^15, so 24-bit multiplies (full rate, with a 32-bit add; a 32-bit multiply takes four times as long) give the
+// same exact products.
+template <typename EdgeT>
+__device__ inline EdgeT edge_mul(int32_t a, int32_t b) {
+    if constexpr (sizeof(EdgeT) == 4) return __mul24(a, b);
+    else return EdgeT(a) * EdgeT(b);
+}
+
 // One row of a record inside the bin: E_k(x) for the three edges advances by 256 * A_k per pixel
 // (exact integer steps; EdgeT = int32_t unless the record is wide), depth is the FP32 plane rule of
 // setup, and covered pixels merge into the LDS row with atomic max (64-bit depth | id + 1 words in
@@ -205,7 +213,7 @@ __device__ inline void raster_row(const TriRec& r, uint32_t meta, int ox, int oy
     for (int k = 0; k < 3; ++k) {
         const int n = k == 2 ? 0 : k + 1;
         const int32_t A = Y[n] - Y[k], B = X[k] - X[n];
-        f[k] = EdgeT(A) * EdgeT(Px - X[k]) + EdgeT(B) * EdgeT(Py - Y[k]) - EdgeT((meta >> k) & 1u);
+        f[k] = edge_mul<EdgeT>(A, Px - X[k]) + edge_mul<EdgeT>(B, Py - Y[k]) - EdgeT((meta >> k) & 1u);
         step[k] = EdgeT(A) * EdgeT(256);
     }
     const float fy = float(Py - r.Y0);
@@ -230,15 +238,18 @@ __device__ inline void raster_row_ms(const TriRec& r, uint32_t meta, int ox, int
     const int32_t X[3] = {r.X0, r.X1, r.X2}, Y[3] = {r.Y0, r.Y1, r.Y2};
     const int32_t Py = (oy + y) * 256 + 128;
     int32_t Px = (ox + bx0) * 256 + 128;
-    EdgeT f[3], step[3], d[4][3];
+    // the locations lie symmetrically about the centre: sample 3's offset is minus sample 0's, 2's minus 1's
+    static_assert(msaa_x(3) + msaa_x(0) == 256 && msaa_y(3) + msaa_y(0) == 256 && msaa_x(2) + msaa_x(1) == 256 &&
+                      msaa_y(2) + msaa_y(1) == 256, "symmetric sample locations");
+    EdgeT f[3], step[3], d[2][3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const int n = k == 2 ? 0 : k + 1;
         const int32_t A = Y[n] - Y[k], B = X[k] - X[n];
-        f[k] = EdgeT(A) * EdgeT(Px - X[k]) + EdgeT(B) * EdgeT(Py - Y[k]) - EdgeT((meta >> k) & 1u);
+        f[k] = edge_mul<EdgeT>(A, Px - X[k]) + edge_mul<EdgeT>(B, Py - Y[k]) - EdgeT((meta >> k) & 1u);
         step[k] = EdgeT(A) * EdgeT(256);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) d[s][k] = EdgeT(A) * EdgeT(msaa_x(s) - 128) + EdgeT(B) * EdgeT(msaa_y(s) - 128);
+        for (int s = 0; s < 2; ++s) d[s][k] = edge_mul<EdgeT>(A, msaa_x(s) - 128) + edge_mul<EdgeT>(B, msaa_y(s) - 128);
     }
     float fy[4];
 #pragma unroll
@@ -250,7 +261,8 @@ __device__ inline void raster_row_ms(const TriRec& r, uint32_t meta, int ox, int
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             zb[s] = 0u;
-            if (((f[0] + d[s][0]) | (f[1] + d[s][1]) | (f[2] + d[s][2])) >= 0) {
+            auto at = [&](int k) { return s < 2 ? f[k] + d[s & 1][k] : f[k] - d[(3 - s) & 1][k]; };
+            if ((at(0) | at(1) | at(2)) >= 0) {
                 float z = fmaf(r.dzdy, fy[s], fmaf(r.dzdx, float(Px + msaa_x(s) - 128 - r.X0), r.z0));
                 z = fminf(fmaxf(z, 0.0f), 1.0f);
                 zb[s] = fbits(z) & 0x7fffffffu;
@@ -263,50 +275,83 @@ __device__ inline void raster_row_ms(const TriRec& r, uint32_t meta, int ox, int
     }
 }
 
+// LDS of one work item's records.  Tasks are rows, and with 4 samples row segments of eight pixels: a wave takes as
+// long as its longest task, and a pixel costs four times as much there (k_raster<32, 4> with whole rows and with
+// segments: 79 and 68 us at 1600 x 900; with one sample the segments' own cost outweighs it: 55 and 60 us for the
+// views of a 2560 x 1440 frame with four cascades).  A task finds its record by a bit per task (set where a record's
+// tasks begin) and the count of records that began before the 64 tasks of its word; a table of one byte a task took
+// a serial store loop per record and twice the space (58 us for the same views).
+template <int T, int N>
+struct RasterLds {
+    static constexpr int kSeg = N == 4 ? 8 : T, kSegs = T / kSeg;
+    static constexpr uint32_t kChunkRecs = 128;  // records staged at a time
+    static constexpr uint32_t kWords = kChunkRecs * T * kSegs / 64;
+    TriRec recs[kChunkRecs];  // the staged records that touch the tile
+    unsigned long long begins[kWords];
+    uint8_t before[kWords];
+    uint16_t first[kChunkRecs];  // a record's first task
+    uint32_t scan[4];
+};
+
 // The records of one work item through the bin's LDS tile.  Every thread loads one record of the
 // item (its box clipped to the bin, its raster flags computed) in one round of loads; the records
 // then go through LDS kChunkRecs at a time, each chunk staged by its own threads.  A staged
-// record's rows become tasks (a prefix sum numbers them and each record writes its index into the
-// task-owner table), and every thread takes tasks in turn, so small and large triangles spread
-// evenly over the workgroup.
-template <int T, class Op>
-__device__ inline void raster_item(const Op& op, TriRec* chunk_recs, uint8_t* owner, uint32_t* row_start,
-                                   uint32_t* scan_lds, bool have, uint4 w0, uint4 w1, uint4 w2, uint32_t n, int ox,
-                                   int oy) {
+// record's row segments become tasks (a prefix sum numbers them) and every thread takes tasks in
+// turn, so small and large triangles spread evenly over the workgroup.
+template <int T, class Lds, class Op>
+__device__ inline void raster_item(const Op& op, Lds& lds, bool have, uint4 w0, uint4 w1, uint4 w2, uint32_t n,
+                                   int ox, int oy) {
+    constexpr uint32_t kChunkRecs = Lds::kChunkRecs;
     static_assert(kItemRecs == 256 && kItemRecs % kChunkRecs == 0, "one record per thread");
-    uint32_t my_rows = 0;
+    static_assert(kChunkRecs * T * Lds::kSegs < 65536u && kChunkRecs < 256u && Lds::kSegs <= 4, "task numbers of 16 bits");
+    uint32_t my_tasks = 0;
     if (have) {
         const int bx0 = max(int(w2.z & 0xffffu), ox) - ox, bx1 = min(int(w2.z >> 16), ox + T - 1) - ox;
         const int by0 = max(int(w2.w & 0xffffu), oy) - oy, by1 = min(int(w2.w >> 16), oy + T - 1) - oy;
         if (bx0 <= bx1 && by0 <= by1) {
-            my_rows = uint32_t(by1 - by0 + 1);
+            my_tasks = uint32_t(by1 - by0 + 1) * (uint32_t(bx1 - bx0) / Lds::kSeg + 1u);
             // the staged copy keeps the clipped box in bbx and the raster flags in bby
             w2.z = uint32_t(bx0) | (uint32_t(bx1) << 8) | (uint32_t(by0) << 16);
             w2.w = record_meta(int32_t(w0.x), int32_t(w0.y), int32_t(w0.z), int32_t(w0.w), int32_t(w1.x),
                                int32_t(w1.y));
         }
     }
-    const uint32_t slot = threadIdx.x % kChunkRecs;
     for (uint32_t c = 0; c * kChunkRecs < n; ++c) {
-        const bool stager = threadIdx.x / kChunkRecs == c;
-        const uint32_t rows = stager ? my_rows : 0u;
-        if (rows) {
-            uint4* dst = reinterpret_cast<uint4*>(chunk_recs + slot);
+        const uint32_t tasks = threadIdx.x / kChunkRecs == c ? my_tasks : 0u;
+        for (uint32_t i = threadIdx.x; i < Lds::kWords; i += 256) lds.begins[i] = 0ull;
+        // one prefix sum numbers the tasks (low half) and the records that have any (high half); it synchronises, and
+        // the barrier after the staging comes before the next chunk's scan writes
+        uint32_t sums;
+        const uint32_t excl = block_exclusive_scan<false>(tasks | (tasks ? 0x10000u : 0u), lds.scan, sums);
+        const uint32_t total = sums & 0xffffu;
+        if (tasks) {
+            const uint32_t f = excl & 0xffffu, rank = excl >> 16, last = f + tasks - 1u;
+            uint4* dst = reinterpret_cast<uint4*>(lds.recs + rank);
             dst[0] = w0;
             dst[1] = w1;
             dst[2] = w2;
+            lds.first[rank] = uint16_t(f);
+            atomicOr(&lds.begins[f >> 6], 1ull << (f & 63u));
+            if ((f & 63u) == 0u) lds.before[f >> 6] = uint8_t(rank);
+            for (uint32_t w = (f >> 6) + 1u; w <= last >> 6; ++w) lds.before[w] = uint8_t(rank + 1u);
         }
-        uint32_t total_rows;
-        // synchronises; the barrier after the owner table comes before the next chunk's scan writes
-        const uint32_t first = block_exclusive_scan<false>(rows, scan_lds, total_rows);
-        if (stager) row_start[slot] = first;
-        for (uint32_t j = 0; j < rows; ++j) owner[first + j] = uint8_t(slot);
         __syncthreads();
-        for (uint32_t task = threadIdx.x; task < total_rows; task += 256) {
-            const uint32_t k = owner[task];
-            const TriRec q = chunk_recs[k];
-            const int bx0 = int(q.bbx & 0xffu), bx1 = int((q.bbx >> 8) & 0xffu);
-            const int y = int((q.bbx >> 16) & 0xffu) + int(task - row_start[k]);
+        for (uint32_t task = threadIdx.x; task < total; task += 256) {  // a wave's 64 tasks share a word
+            const unsigned long long b = lds.begins[task >> 6];
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(uint32_t(b >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(b), 0u));
+            const uint32_t k = lds.before[task >> 6] + below + (uint32_t(b >> lane_id()) & 1u) - 1u;
+            const TriRec q = lds.recs[k];
+            int bx0 = int(q.bbx & 0xffu), bx1 = int((q.bbx >> 8) & 0xffu);
+            const uint32_t j = task - lds.first[k];
+            uint32_t row = j;
+            if constexpr (Lds::kSegs > 1) {
+                const uint32_t segs = uint32_t(bx1 - bx0) / Lds::kSeg + 1u;
+                // j / segs; by three as a product, exact below 512
+                row = segs == 1u ? j : segs == 2u ? j >> 1 : segs == 3u ? (j * 171u) >> 9 : j >> 2;
+                bx0 += int(j - row * segs) * Lds::kSeg;
+                bx1 = min(bx1, bx0 + Lds::kSeg - 1);
+            }
+            const int y = int((q.bbx >> 16) & 0xffu) + int(row);
             if constexpr (Op::kSamples == 4) {
                 if (q.bby & kMetaWide)
                     raster_row_ms<int64_t>(q, q.bby, ox, oy, y, bx0, bx1, op);

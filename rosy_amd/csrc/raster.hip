@@ -1029,10 +1029,7 @@ __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n
                                                 uint32_t* report) {
     constexpr int S = T + 1;  // padded row stride (words)
     __shared__ unsigned long long tile[N * T * S];  // camera views: one plane per sample
-    __shared__ TriRec chunk_recs[kChunkRecs];
-    __shared__ uint8_t owner[kChunkRecs * T];  // task (row) -> record of the chunk
-    __shared__ uint32_t row_start[kChunkRecs];  // exclusive prefix of row counts
-    __shared__ uint32_t scan_lds[4];
+    __shared__ RasterLds<T, N> lds;
 
     // One workgroup per item.  The grid is sized from the last frame's item count (the count of
     // this frame is known only on the device): the bin scan flags a frame with more items than
@@ -1040,6 +1037,7 @@ __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n
     // beside the count (blockIdx.x < gridDim.x <= the table's capacity).
     const uint32_t n_items = totals[3];
     const uint4 it = items[blockIdx.x];
+    const uint32_t my_base = lane_id() < n_views ? views[lane_id()].tile_base : 0u;
     // the last workgroup (past the items, as a rule) also reports the frame's counters
     if (report && blockIdx.x + 1u == gridDim.x) report_counters(report, counters, n_views, totals);
     // (the test reads the item too, which keeps its load beside the count's instead of after the
@@ -1053,8 +1051,8 @@ __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n
     const uint32_t n = end > off ? end - off : 0u;  // at most kItemRecs
     const uint32_t ri = threadIdx.x < n ? lists[off + threadIdx.x] : 0xffffffffu;
     const uint32_t bin = it.x;
-    uint32_t view = 0;
-    while (view + 1 < n_views && views[view + 1].tile_base <= bin) ++view;
+    // the last view whose first bin is not past this one (bins are numbered view by view)
+    const uint32_t view = uint32_t(__builtin_popcountll(__ballot(lane_id() < n_views && my_base <= bin))) - 1u;
     const ViewGPU V = views[view];
     if (V.blend) return;  // blend views are drawn by the blended pass (k_blend)
     const uint32_t local_bin = bin - V.tile_base;
@@ -1072,7 +1070,7 @@ __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n
     if (V.is_shadow) {
         uint32_t* t32 = reinterpret_cast<uint32_t*>(tile);
         for (int p = threadIdx.x; p < T * S; p += 256) t32[p] = 0u;
-        raster_item<T>(ShadowFrag<T>{t32}, chunk_recs, owner, row_start, scan_lds, have, w0, w1, w2, n, ox, oy);
+        raster_item<T>(ShadowFrag<T>{t32}, lds, have, w0, w1, w2, n, ox, oy);
         __syncthreads();  // tile complete (and cleared, for an item without records)
         uint32_t* out = reinterpret_cast<uint32_t*>(out_addr);
         for (int p = threadIdx.x; p < T * T; p += 256) {
@@ -1087,9 +1085,9 @@ __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n
     } else {
         for (int p = threadIdx.x; p < N * T * S; p += 256) tile[p] = 0ull;
         if constexpr (N == 4)
-            raster_item<T>(CameraFragMS<T>{tile}, chunk_recs, owner, row_start, scan_lds, have, w0, w1, w2, n, ox, oy);
+            raster_item<T>(CameraFragMS<T>{tile}, lds, have, w0, w1, w2, n, ox, oy);
         else
-            raster_item<T>(CameraFrag<T>{tile}, chunk_recs, owner, row_start, scan_lds, have, w0, w1, w2, n, ox, oy);
+            raster_item<T>(CameraFrag<T>{tile}, lds, have, w0, w1, w2, n, ox, oy);
         __syncthreads();
         unsigned long long* out = reinterpret_cast<unsigned long long*>(out_addr);
         const size_t plane = size_t(width) * height;

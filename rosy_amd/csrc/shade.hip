@@ -806,10 +806,7 @@ __global__ __launch_bounds__(256) void k_blend_collect(const BlendLaunch B) {
     constexpr uint32_t kKeyMask = N == 4 ? 0x0fffffffu : 0xffffffffu;
     __shared__ uint32_t opaque[N * U * S], count[U * S], cursor[U * S];
     __shared__ uint32_t lds_keys[kLdsFrags];
-    __shared__ TriRec chunk_recs[kChunkRecs];
-    __shared__ uint8_t owner[kChunkRecs * U];
-    __shared__ uint32_t row_start[kChunkRecs];
-    __shared__ uint32_t scan_lds[4];
+    __shared__ RasterLds<U, N> lds;
     __shared__ uint32_t base_lds;
 
     const uint32_t bin = B.views[B.first_blend].tile_base + blockIdx.x / Q;
@@ -845,7 +842,7 @@ __global__ __launch_bounds__(256) void k_blend_collect(const BlendLaunch B) {
             const bool have = ri < B.rec_cap_total;
             const uint4* src = reinterpret_cast<const uint4*>(B.recs + (have ? ri : 0u));
             const uint4 w0 = src[0], w1 = src[1], w2 = src[2];
-            raster_item<U>(op, chunk_recs, owner, row_start, scan_lds, have, w0, w1, w2, n, ox, oy);
+            raster_item<U>(op, lds, have, w0, w1, w2, n, ox, oy);
         }
     };
     if constexpr (N == 4) sweep(CountFragMS<U>{count, opaque});  // ends on a barrier
@@ -853,7 +850,7 @@ __global__ __launch_bounds__(256) void k_blend_collect(const BlendLaunch B) {
 
     const uint32_t n = count[pi];
     uint32_t total;
-    const uint32_t first = block_exclusive_scan(n, scan_lds, total);
+    const uint32_t first = block_exclusive_scan(n, lds.scan, total);
     cursor[pi] = first;
     if (threadIdx.x == 0) base_lds = atomicAdd(&B.counters[B.first_blend * kCtrPerView + kCtrFrags], total);
     __syncthreads();
@@ -886,7 +883,7 @@ __global__ __launch_bounds__(256) void k_blend_collect(const BlendLaunch B) {
     uint32_t layer_base = base;
     for (uint32_t a = 0;; ++a) {
         uint32_t in_layer;
-        const uint32_t rank = block_exclusive_scan(a < n ? 1u : 0u, scan_lds, in_layer);
+        const uint32_t rank = block_exclusive_scan(a < n ? 1u : 0u, lds.scan, in_layer);
         if (in_layer == 0u) break;
         if (a < n) B.frags[layer_base + rank] = make_uint4(l[a] & kKeyMask, xy, sview, base + first + a);
         layer_base += in_layer;
