@@ -70,6 +70,45 @@ __device__ inline float cmp_tap(GlobalPtr<const float> map, int S, float u, floa
            (1 - ax) * ay * (ref >= t01 ? 1.f : 0.f) + ax * ay * (ref >= t11 ? 1.f : 0.f);
 }
 
+// The two texel rows of a tap, each its two texels from one eight-byte load (maps of two texels a side or more): a
+// texel past an edge is the edge's own.  Five taps were twenty loads of a pixel's forty (k_shade 41.5 and 37.7 us at
+// 1920 x 1080 with them and with ten).  Requesting them before the material's texels holds twenty registers through
+// the sampling and costs a wave a SIMD (40.9 us; 94 instead of 82 at 2560 x 1440).
+struct TapTexels {
+    float2 row[2];
+};
+struct __attribute__((packed, aligned(4))) TexelPair {
+    float a, b;
+};
+__device__ inline TapTexels tap_texels(GlobalPtr<const float> map, int S, float u, float v) {
+    const float x = u * float(S) - 0.5f, y = v * float(S) - 0.5f;
+    const int x0 = int(floorf(fminf(fmaxf(x, -2.0f), float(S) + 1.0f)));
+    const int y0 = int(floorf(fminf(fmaxf(y, -2.0f), float(S) + 1.0f)));
+    const int xp = min(max(x0, 0), S - 2);
+    TapTexels t;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int yk = min(max(y0 + k, 0), S - 1);
+        const TexelPair p = *(GlobalPtr<const TexelPair>)(map + (size_t(yk) * S + xp));
+        t.row[k] = make_float2(p.a, p.b);
+    }
+    return t;
+}
+// cmp_tap on texels already requested.
+__device__ inline float cmp_texels(const TapTexels& t, int S, float u, float v, float ref) {
+    const float x = u * float(S) - 0.5f, y = v * float(S) - 0.5f;
+    const float fx0 = floorf(fminf(fmaxf(x, -2.0f), float(S) + 1.0f));
+    const float fy0 = floorf(fminf(fmaxf(y, -2.0f), float(S) + 1.0f));
+    const float ax = x - fx0, ay = y - fy0;
+    const int x0 = int(fx0);
+    // left of the map both texels are the first of the pair, right of it both the second
+    const bool left = x0 < 0, right = x0 > S - 2;
+    const float t00 = right ? t.row[0].y : t.row[0].x, t10 = left ? t.row[0].x : t.row[0].y;
+    const float t01 = right ? t.row[1].y : t.row[1].x, t11 = left ? t.row[1].x : t.row[1].y;
+    return (1 - ax) * (1 - ay) * (ref >= t00 ? 1.f : 0.f) + ax * (1 - ay) * (ref >= t10 ? 1.f : 0.f) +
+           (1 - ax) * ay * (ref >= t01 ? 1.f : 0.f) + ax * ay * (ref >= t11 ? 1.f : 0.f);
+}
+
 // Frame constants of a shading launch.  The scene data is read through the constant address space
 // (scalar loads, shared by the waves of a CU).  The sRGB table and the cascades (selected per
 // pixel) are copied into LDS at the start of each workgroup: shared_request issues the loads (one
@@ -152,18 +191,20 @@ __device__ Varyings pixel_varyings(SceneP sd, const rsy_position* const v[3], GP
         if (sd->flip_tangents[3] == 1) nt.w = -nt.w;
         const f3 n = mk(r0.w, r1.x, r1.y);
         const f3 t = mk(nt.x, nt.y, nt.z);
-        f3 bt = cross(n, t) * nt.w;
-        if (sd->ensure_orthogonal_bitangent == 1) {
-            const f3 np = bt * dot(n, bt);
-            const f3 on = normalize(n - np);
-            const f3 tp = np - bt * dot(t, bt);
-            const f3 ot = normalize(t - tp);
-            bt = cross(on, ot) * nt.w;
+        if (sd->fragment_output == 7) {  // the only output that shows the bitangent itself (six registers less elsewhere)
+            f3 bt = cross(n, t) * nt.w;
+            if (sd->ensure_orthogonal_bitangent == 1) {
+                const f3 np = bt * dot(n, bt);
+                const f3 on = normalize(n - np);
+                const f3 tp = np - bt * dot(t, bt);
+                const f3 ot = normalize(t - tp);
+                bt = cross(on, ot) * nt.w;
+            }
+            B = B + bt * w[k];
         }
         P = P + mk(r0.x, r0.y, r0.z) * w[k];
         N = N + n * w[k];
         Tn = Tn + t * w[k];
-        B = B + bt * w[k];
         sigma += nt.w * w[k];
         col.x += r2.z * w[k];
         col.y += r2.w * w[k];
@@ -408,7 +449,11 @@ __device__ __forceinline__ Fragment shade_pixel(const ShadeLaunch& L, const Shad
         else return sample_tex(t, smp, tu, tv, lut);
     };
     const float4 csm = bv.csm;
-
+    const bool shadowed = sd->light_enabled > 0 && sd->shadows_enabled == 1 && cascade >= 0;
+    const float so = 0.00025f;
+    const float tap_u[5] = {csm.x - so, csm.x + so * 2.f, csm.x, csm.x + so * 2.f, csm.x - so * 2.f};
+    const float tap_v[5] = {csm.y - so, csm.y, csm.y + so * 2.f, csm.y + so * 2.f, csm.y - so * 2.f};
+    const bool five_taps = shadowed && L.pcf_mode != RSY_PCF_GRID_3X3 && S.casc[cascade].size >= 2u;
     const f3 ambient = mk(sd->ambient_color[0], sd->ambient_color[1], sd->ambient_color[2]);
     float4 out = bcol;
     float4 image = out;
@@ -516,24 +561,29 @@ __device__ __forceinline__ Fragment shade_pixel(const ShadeLaunch& L, const Shad
     if (set) out = make_float4(c3.x, c3.y, c3.z, alpha);
     float shadow = 1.f;
     if (sd->light_enabled > 0) {
-        if (sd->shadows_enabled == 1 && cascade >= 0) {
+        if (five_taps) {
+            TapTexels taps[5];
+            const GlobalPtr<const float> map = gmem(S.casc[cascade].map);
+            const int Sz = int(S.casc[cascade].size);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) taps[k] = tap_texels(map, Sz, tap_u[k], tap_v[k]);
+            float r = 0.f;
+#pragma unroll
+            for (int k = 0; k < 5; ++k) r += cmp_texels(taps[k], Sz, tap_u[k], tap_v[k], csm.z);
+            shadow = r * (1.0f / 5.0f);
+        } else if (shadowed) {
             const ShadeCascade& C = S.casc[cascade];
             const GlobalPtr<const float> map = gmem(C.map);
             const int Sz = int(C.size);
+            float r = 0.f;
             if (L.pcf_mode == RSY_PCF_GRID_3X3) {
-                float r = 0.f;
                 const float inv = 1.0f / float(Sz);
                 for (int j = -1; j <= 1; ++j)
                     for (int i = -1; i <= 1; ++i) r += cmp_tap(map, Sz, csm.x + float(i) * inv, csm.y + float(j) * inv, csm.z);
                 shadow = r * (1.0f / 9.0f);
-            } else {
-                const float so = 0.00025f;
-                float r = 0.f;
-                r += cmp_tap(map, Sz, csm.x - so, csm.y - so, csm.z);
-                r += cmp_tap(map, Sz, csm.x + so * 2.f, csm.y, csm.z);
-                r += cmp_tap(map, Sz, csm.x, csm.y + so * 2.f, csm.z);
-                r += cmp_tap(map, Sz, csm.x + so * 2.f, csm.y + so * 2.f, csm.z);
-                r += cmp_tap(map, Sz, csm.x - so * 2.f, csm.y - so * 2.f, csm.z);
+            } else {  // a map of one texel
+#pragma unroll 1
+                for (int k = 0; k < 5; ++k) r += cmp_tap(map, Sz, tap_u[k], tap_v[k], csm.z);
                 shadow = r * (1.0f / 5.0f);
             }
         }
@@ -583,8 +633,11 @@ __device__ inline bool wave_uniform(uint32_t v) {
     return __builtin_amdgcn_ballot_w64(v != v0) == 0ull;
 }
 
+// Bound by the latency of its chain of loads (visibility word, records, vertices, texels and shadow taps), so waves in
+// flight count for more than registers: 96 of them and a few spilled words give five a SIMD (35.5 us at 1920 x 1080, 219
+// for four cameras with the decoder) where 108 to 114 give four (37 and 237); six a SIMD spill too much (46 and 302).
 template <bool kNeural, bool kLod>
-__global__ __launch_bounds__(256) void k_shade(ShadeLaunch L) {
+__global__ __launch_bounds__(256, 5) void k_shade(ShadeLaunch L) {
     __shared__ ShadeShared S;
     const SharedWords sw = shared_request(L);
 
@@ -659,8 +712,9 @@ __global__ __launch_bounds__(256) void k_shade(ShadeLaunch L) {
 // by its edge pixels), their colours kept in LDS; each pixel then writes the average of its four
 // samples (and, with a blended pass to follow, the sample colours).  The debug shadow factor is
 // that of sample 0's primitive.
+// Four waves a SIMD for the reason given at k_shade: 49 us at 1600 x 900 instead of 55.5 with three.
 template <bool kNeural, bool kLod>
-__global__ __launch_bounds__(256) void k_shade_ms(ShadeLaunch L) {
+__global__ __launch_bounds__(256, 4) void k_shade_ms(ShadeLaunch L) {
     __shared__ ShadeShared S;
     __shared__ uint16_t jobs[1024];       // pixel (thread) << 2 | first sample of the primitive
     __shared__ float4 job_color[1024];
@@ -892,7 +946,8 @@ __global__ __launch_bounds__(256) void k_blend_collect(const BlendLaunch B) {
 
 // Every fragment of the frame shaded at its pixel centre (a grid-stride loop over the count the
 // collection left), its colour stored at the index its record names.  Records of sub-tiles that ran
-// out of space have key 0 and are skipped.
+// out of space have key 0 and are skipped.  (112 registers, four waves a SIMD: 49 us for the translucent 1080p frame;
+// held to five waves it spills more than it gains, 53 us.)
 template <bool kLod>
 __global__ __launch_bounds__(256) void k_blend_shade(const BlendLaunch B, const ShadeLaunch L) {
     __shared__ ShadeShared S;

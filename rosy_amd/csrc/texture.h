@@ -137,7 +137,7 @@ __device__ __forceinline__ float4 sample_tex_lod(const TexRef& t, const SamplerS
 // The three maps of a packed material at one place, with the arithmetic of sample_tex on each of them.  Shading is
 // bound by the lines its texels lie on: one by one, a pixel reads two rows of each of three images (six lines of 128
 // bytes) through twelve loads and computes its addresses and weights three times; packed, it reads the eight-byte texels
-// of a 2 x 2 square out of 4 x 4 tiles (1.6 lines) in four loads.  Measured, one by one and packed: k_shade 60 and 41 us
+// of a 2 x 2 square out of 4 x 4 tiles (1.6 lines) in four loads.  Measured, one by one and packed (the rest of the kernels as they then were): k_shade 60 and 41 us
 // at 1920 x 1080 (127 and 87 at 2560 x 1440), k_shade_ms with level of detail 104 and 54 us at 1366 x 768,
 // k_blend_shade 87 and 53 us.
 struct PackSample {
