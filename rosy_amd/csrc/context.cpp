@@ -1213,6 +1213,7 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     for (auto& t : table) c->tex_channels.push_back(t.channels);
     c->h_materials.assign(materials, materials + n_materials);
     c->h_tex_table = table;
+    c->h_packs = packs;
     c->h_samplers.assign(samplers, samplers + n_samplers);
     // the draws' sampler flags follow the materials: refreshed in place, so that the allocation-free
     // render path keeps working after a material change

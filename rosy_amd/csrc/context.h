@@ -214,6 +214,7 @@ struct rsy_ctx {
     std::vector<rsy_gpu_material> h_materials;
     std::vector<rsy::TexGPU> h_tex_table;
     std::vector<rsy_sampler> h_samplers;
+    std::vector<rsy::PackGPU> h_packs;  // per material
     std::vector<uint8_t> tex_opaque;  // four-channel texture whose alpha is 255 everywhere
     rsy::DevBuf tex_staging;          // BC7 blocks on their way to the decoder
     rsy::DevBuf tex_jobs, tex_flags;  // the upload kernels' images and alpha-test results

@@ -208,6 +208,8 @@ struct NmTrainLaunch {
     const TexGPU* maps;  // [slots][3]: each slot's albedo, normal and metallic-roughness records
     uint32_t n_slots;
     const uint8_t* texels;
+    const PackGPU* packs;  // [slots]: the same maps as one packed image, or levels 0
+    const uint8_t* packed;
     const float* srgb_lut;
     uint32_t L, log2L;
     uint32_t log2R;   // region side 2^log2R cells

@@ -117,8 +117,21 @@ __device__ inline void row_pair(const uint8_t* map, const Taps& t, int row, uint
         second = q.b;
     }
 }
-__device__ inline StepTexels step_texels(const uint8_t* texels, const TexGPU& ta, const TexGPU& tn, const TexGPU& tm,
-                                         float u, float v) {
+__device__ inline StepTexels step_texels(const uint8_t* texels, const uint8_t* packed, const PackGPU& pk, const TexGPU& ta,
+                                         const TexGPU& tn, const TexGPU& tm, float u, float v) {
+    if (pk.levels != 0u) {  // the maps as one packed image (a decoded material's samplers repeat)
+        const PackTaps q = pack_taps(reinterpret_cast<const uint2*>(packed + pk.offset), int(pk.width), int(pk.height),
+                                     2u << kPackWrapS | 2u << kPackWrapT, u, v);
+        StepTexels p;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            p.a[k] = q.t[k].x;
+            p.n[k] = q.t[k].y & 0xffffu;
+            p.m[k] = q.t[k].y >> 16;
+            p.wa[k] = p.wn[k] = p.wm[k] = q.w[k];
+        }
+        return p;
+    }
     const Taps a = taps_of(ta, u, v);  // maps of one extent (a uniform test) share their footprint
     Taps n = a, m = a;
     if (tn.width != ta.width || tn.height != ta.height) n = taps_of(tn, u, v);
@@ -215,15 +228,17 @@ __global__ __launch_bounds__(256) void k_nm_tables(const float* mlp, float* tabl
 // A step has 65,536 samples by default: one sample wave on each of the chip's 1,024 SIMDs, so the kernel's
 // time is the length of one wave's chain: the step counter, the slot's map records, the texels (each
 // launch starts with a cold L2: 2,000 cycles a hop), the MLP, its gradient.
-// - Loads that depend on nothing else go out together at the start, the texels in pairs; the cell waves
-//   load the region's Adam state, whose latents the samples read from LDS.
+// - Loads that depend on nothing else go out together at the start; the cell waves load the region's Adam
+//   state, whose latents the samples read from LDS.
+// - A sample's texels come from its material's packed image: four loads on 1.6 lines (14.4 us a step) instead of
+//   six loads on six lines (18.7 us: the texel pages and lines of 65,536 samples), which maps that cannot be packed keep.
 // - The MLP runs in registers on the matrix cores (its weights were read from LDS, one wait per hidden unit).
 // - Its gradient, a product over the samples, is one matrix instruction per sample and wave from
 //   records in LDS: 256 multiply-adds in sample order for every parameter, as the scalar loops had it
 //   (three dot products of 256 LDS pairs a thread, 20,000 cycles), 29 cycles apart.
 // - Latent gradients were 32 LDS float atomics a sample (20,000 cycles): the samples are sorted by cell
 //   while their texels are on the way, and the cell waves sum them and apply Adam beside the MLP gradient.
-// 65,536 samples of 16 materials: 47 us before, 18 us; the MLP's update 6.2 and 5.3 us.
+// 65,536 samples of 16 materials: 47 us before, 14.4 us; the MLP's update 6.2 and 5.3 us.
 template <bool kExplicit>
 __global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
     constexpr uint32_t kMaxCells = kMaxR * kMaxR, kCellsPerThread = kMaxCells / 256;
@@ -271,12 +286,14 @@ __global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
     const size_t grid_base = size_t(slot) * L * L;
     auto cell_of = [&](uint32_t cx, uint32_t cy) { return grid_base + size_t((ry + cy) & Lm) * L + ((rx + cx) & Lm); };
     TexGPU ta{}, tn{}, tm{};
+    PackGPU pk{};
     float4 adam[6] = {};  // a cell wave: the Adam state of the thread's first cell, and the step's factors
     float bc1 = 1.f, bc2 = 1.f, lr = 0.f;
     if (sampler) {
         ta = T.maps[3 * slot];
         tn = T.maps[3 * slot + 1];
         tm = T.maps[3 * slot + 2];
+        pk = T.packs[slot];
     } else {
         const float srgb = T.srgb_lut[tid];
         if (!kExplicit && tid < cells) {
@@ -360,7 +377,7 @@ __global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
 #pragma unroll
                 for (int c = 0; c < kNmOut; ++c) tgt[c] = T.ex_target[kNmOut * size_t(s_base + q) + c];
             } else {
-                px = step_texels(T.texels, ta, tn, tm, u, v);
+                px = step_texels(T.texels, T.packed, pk, ta, tn, tm, u, v);
             }
         }
         __syncthreads();  // counts cleared, tables written, the last chunk's records read

@@ -28,7 +28,7 @@ struct NeuralState {
     std::vector<uint32_t> block_base;  // evaluation tiles per slot (prefix, n_slots + 1)
     uint32_t max_tiles = 0;            // of the largest slot
     bool any_same = false, any_other = false;  // some slot's maps share one extent / differ in size
-    DevBuf slots_d, maps_d, slot_of_d, active_d, block_base_d;
+    DevBuf slots_d, maps_d, packs_d, slot_of_d, active_d, block_base_d;
     DevBuf lat, lat_m, lat_v, mlp, mlp_m, mlp_v, tables, partial, step_d, loss_d, lat16, weights_d, eval_partial, eval_sum;
     DevBuf tmp[5];
     uint32_t n_wg = 0, spw = 0;
@@ -136,6 +136,8 @@ NmTrainLaunch train_args(rsy_ctx* c, NeuralState* n) {
     T.maps = n->maps_d.as<TexGPU>();
     T.n_slots = uint32_t(n->slots.size());
     T.texels = c->texels.as<uint8_t>();
+    T.packs = n->packs_d.as<PackGPU>();
+    T.packed = c->packed.as<uint8_t>();
     T.srgb_lut = c->srgb_lut.as<float>();
     T.L = n->L;
     T.log2L = n->log2L;
@@ -240,6 +242,7 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     HIP_TRY(c, hipEventCreate(&n->ev1), "event");
     HIP_TRY(c, n->slots_d.ensure(std::max<size_t>(1, ns) * sizeof(NmSlot)), "allocate decoder");
     HIP_TRY(c, n->maps_d.ensure(std::max<size_t>(1, ns) * 3 * sizeof(TexGPU)), "allocate decoder");
+    HIP_TRY(c, n->packs_d.ensure(std::max<size_t>(1, ns) * sizeof(PackGPU)), "allocate decoder");
     HIP_TRY(c, n->slot_of_d.ensure(std::max<size_t>(1, nm) * 4), "allocate decoder");
     HIP_TRY(c, n->active_d.ensure(std::max<size_t>(1, nm) * 4), "allocate decoder");
     HIP_TRY(c, n->block_base_d.ensure((ns + 1) * 4), "allocate decoder");
@@ -260,6 +263,9 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     HIP_TRY(c, n->eval_sum.ensure(std::max<size_t>(1, ns) * 8), "allocate decoder");
     if (ns) {
         std::vector<TexGPU> maps;
+        std::vector<PackGPU> packs;
+        for (const NmSlot& sl : n->slots) packs.push_back(c->h_packs[sl.material]);
+        HIP_TRY(c, hipMemcpy(n->packs_d.p, packs.data(), packs.size() * sizeof(PackGPU), hipMemcpyHostToDevice), "upload");
         for (const NmSlot& sl : n->slots)
             for (uint32_t k : {sl.albedo, sl.normal, sl.mr}) maps.push_back(c->h_tex_table[k]);
         HIP_TRY(c, hipMemcpy(n->slots_d.p, n->slots.data(), ns * sizeof(NmSlot), hipMemcpyHostToDevice), "upload");
