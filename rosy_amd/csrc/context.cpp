@@ -323,7 +323,7 @@ rsy_result plan_layout(rsy_ctx* c, const std::vector<FrameViewDesc>& views, uint
         L.tblocks.swap(paired);
     }
     interleave_views(L.tblocks);  // (the transform keeps view order: its output writes stream per view)
-    // output clears: in the view's setup blocks when each block's share is small, else a fill launch
+    // output clears: in the view's setup blocks when each block's share is small, else in k_clip
     std::vector<uint32_t> view_blocks(L.vg.size(), 0u);
     for (const BlockEntry& b : L.tblocks) ++view_blocks[b.view];
     for (size_t v = 0; v < L.vg.size(); ++v) {
@@ -625,12 +625,6 @@ rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool ca
     g.clip_blocks = 128;
     g.total_bins = L.total_bins;
     HIP_TRY(c, launch_geometry(g, s), "geometry kernels");
-    // the outputs that the setup blocks do not clear (views with few setup blocks for their size)
-    for (const ViewGPU& v : L.vg)
-        if (!v.blend && !v.setup_clear) {
-            const uint64_t words = uint64_t(v.width) * v.height * (v.is_shadow ? 1u : 2u * v.samples);
-            HIP_TRY(c, launch_fill_u32(reinterpret_cast<uint32_t*>(v.out), uint32_t(words), 0u, s), "clear output");
-        }
     if (timing) HIP_TRY(c, hipEventRecord(c->ev_stage[0], s), "event");
 
     BinLaunch b{};

@@ -19,7 +19,7 @@ constexpr uint32_t kSetupBlockTris = 256;
 // A frame whose setup would take more blocks than this runs two triangles per thread (512 per block).
 constexpr uint32_t kSetupPairBlocks = 8192;
 // A view's setup blocks clear its output when each block's share is at most this many bytes; a view
-// with fewer, larger shares is cleared by a fill launch instead
+// with fewer, larger shares is cleared by k_clip instead
 constexpr uint64_t kSetupClearBytes = 128u << 10;
 
 // The three draw lists of a frame, indexed by ViewGPU::list.
@@ -281,7 +281,6 @@ hipError_t launch_alpha_test(const MipJob* jobs, uint32_t n_jobs, const uint8_t*
 // the packed images of `jobs` (at most max_tiles tiles each over all of their levels)
 hipError_t launch_pack(const PackJob* jobs, uint32_t n_jobs, uint32_t max_tiles, const uint8_t* texels, uint8_t* packed,
                        hipStream_t s);
-hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 hipError_t launch_geometry(const GeometryLaunch& g, hipStream_t s);
 hipError_t launch_binning(const BinLaunch& b, hipStream_t s);
 constexpr uint32_t kScanBlockBins = 1024;    // bins per scan block

@@ -142,10 +142,6 @@ constexpr int kSmallBins = 4;  // records touching at most this many bins are bi
 
 // ---------------------------------------------------------------------------------------------
 
-__global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
-}
-
 // Zeroes two ranges (the per-view counters and the bin counts) in one launch; graph-safe.
 __global__ void k_clear2(uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < na + nb; i += gridDim.x * blockDim.x) {
@@ -394,7 +390,7 @@ __global__ __launch_bounds__(256) void k_setup(const BlockEntry* blocks, const V
         }
     }
     // this block's share of the view's output words, cleared (for a view whose blocks' shares are
-    // small; the host clears the others with a fill launch): k_raster then stores every bin that
+    // small; k_clip clears the others): k_raster then stores every bin that
     // holds records, and merges the items of a split bin into its cleared words.  A view's words are
     // split over its setup blocks in proportion to their record slots, which tile the view's
     // triangles (the stores overlap the block's loads instead of taking a pass of their own)
@@ -561,6 +557,18 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(const ViewGPU* views, con
     const ViewGPU V = views[view];
     uint32_t* ctr = counters + view * kCtrPerView;
     const uint32_t n = min(ctr[kCtrClip], V.clip_cap);
+    // the output of a view whose setup blocks are too few to clear it (a fill launch a view before: with little to
+    // draw, a frame's time is its launches, 72 and 65.5 us at 640 x 360)
+    if (!V.blend && !V.setup_clear) {
+        const uint64_t words = uint64_t(V.width) * V.height * (V.is_shadow ? 1u : 2u * V.samples);
+        struct __attribute__((packed, aligned(4))) Four {  // (a caller's buffer may lie at any word)
+            uint32_t w[4];
+        };
+        const GlobalPtr<Four> q = gmem(reinterpret_cast<Four*>(V.out));
+        for (uint64_t i = blockIdx.x * kClipThreads + threadIdx.x; i < words / 4; i += gridDim.x * kClipThreads)
+            q[i] = Four{};
+        if (blockIdx.x == 0 && threadIdx.x < words % 4) gmem(reinterpret_cast<uint32_t*>(V.out))[words - 1 - threadIdx.x] = 0u;
+    }
     for (uint32_t base = blockIdx.x * kClipThreads; base < n; base += gridDim.x * kClipThreads) {
         const uint32_t q = base + threadIdx.x;
         const bool active = q < n;
@@ -653,7 +661,7 @@ constexpr uint32_t kScanPerThread = 4;
 // larger bin is split into one item per kItemRecs records, and its items merge into the output
 // with device atomic max into the cleared pixels.  Max is order independent, so the result is the
 // same whichever item finishes first.  An empty bin has no item: its pixels keep the clear (made by
-// the view's setup blocks, or by a fill launch for a view with few setup blocks).  One table holds every item as (bin, first list entry, records, split),
+// the view's setup blocks, or by k_clip for a view with few setup blocks).  One table holds every item as (bin, first list entry, records, split),
 // ordered so that the longest items start first and the short ones fill the end of the launch:
 // whole bins with at least kHeavyRecs records, then those with at least kMidRecs, then the split
 // bins' items (each a share of a crowded bin), then the remaining whole bins.
@@ -1108,13 +1116,6 @@ __global__ __launch_bounds__(256) void k_raster(const ViewGPU* views, uint32_t n
 
 // ---------------------------------------------------------------------------------------------
 // Launchers
-
-hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    const uint32_t blocks = min((n + 255) / 256, 4096u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(blocks), dim3(256), 0, s, p, n, v);
-    return hipGetLastError();
-}
 
 hipError_t launch_geometry(const GeometryLaunch& g, hipStream_t s) {
     if (g.n_views == 0) return hipSuccess;
