@@ -619,8 +619,15 @@ __device__ __forceinline__ Fragment shade_pixel(const ShadeLaunch& L, const Shad
     return Fragment{out, shadow, discard};
 }
 
+// The shaded colour, written once and past the caches (as a pixel's visibility word is read), which stay with vertices,
+// texels and shadow map: k_shade 35.3 -> 34.3 us at 1920 x 1080, 76.8 -> 72.4 at 2560 x 1440.
+typedef float f32x4_store __attribute__((ext_vector_type(4)));
+__device__ inline void store_color(const ShadeView& V, size_t o, float4 c) {
+    const f32x4_store v = {c.x, c.y, c.z, c.w};
+    __builtin_nontemporal_store(v, (GlobalPtr<f32x4_store>)(V.color + o));
+}
 __device__ inline void store_fragment(const ShadeView& V, size_t o, const Fragment& f) {
-    gmem(V.color)[o] = f.color;
+    store_color(V, o, f.color);
     if (V.shadow_factor) gmem(V.shadow_factor)[o] = f.shadow;
 }
 
@@ -650,14 +657,14 @@ __global__ __launch_bounds__(256, 5) void k_shade(ShadeLaunch L) {
     const bool inside = x < V.width && y < V.height;
     const size_t o = size_t(y) * V.width + x;
     // the pixel's visibility word is requested beside the workgroup's constants
-    const unsigned long long vis_word = inside ? gmem(V.vis)[o] : 0ull;
+    const unsigned long long vis_word = inside ? __builtin_nontemporal_load(gmem(V.vis) + o) : 0ull;
     shared_store(L, S, sw);
     __syncthreads();
     if constexpr (!kNeural) {
         if (!inside) return;
         const unsigned long long vis = vis_word;
         if (vis == 0ull) {
-            gmem(V.color)[o] = make_float4(L.clear_color[0], L.clear_color[1], L.clear_color[2], L.clear_color[3]);
+            store_color(V, o, make_float4(L.clear_color[0], L.clear_color[1], L.clear_color[2], L.clear_color[3]));
             if (V.shadow_factor) gmem(V.shadow_factor)[o] = 1.f;
             return;
         }
@@ -695,7 +702,7 @@ __global__ __launch_bounds__(256, 5) void k_shade(ShadeLaunch L) {
         if (__builtin_amdgcn_ballot_w64(decode) != 0ull) nm_mlp_wave(static_cast<const NmWeights*>(L.nm_weights), f, dec);
         if (!inside) return;
         if (vis == 0ull) {
-            gmem(V.color)[o] = make_float4(L.clear_color[0], L.clear_color[1], L.clear_color[2], L.clear_color[3]);
+            store_color(V, o, make_float4(L.clear_color[0], L.clear_color[1], L.clear_color[2], L.clear_color[3]));
             if (V.shadow_factor) gmem(V.shadow_factor)[o] = 1.f;
             return;
         }
@@ -822,7 +829,7 @@ __global__ __launch_bounds__(256, 4) void k_shade_ms(ShadeLaunch L) {
             for (int q = 0; q < 4; ++q)
                 if (same & (1u << q)) gmem(V.sample_color)[q * plane + o] = c;
     }
-    gmem(V.color)[o] = make_float4(acc.x * 0.25f, acc.y * 0.25f, acc.z * 0.25f, acc.w * 0.25f);
+    store_color(V, o, make_float4(acc.x * 0.25f, acc.y * 0.25f, acc.z * 0.25f, acc.w * 0.25f));
     if (V.shadow_factor) gmem(V.shadow_factor)[o] = shadow0[threadIdx.x];
 }
 
