@@ -5,9 +5,9 @@
 // sampler's values there (mean squared error over the 7 channels), then applies one Adam update
 // (lr with an optional cosine decay, beta1, beta2, eps) to the latents it touched and to the shared MLP.  Samples are drawn per
 // workgroup inside a region of 2^log2R x 2^log2R latent cells of one material, positioned so that
-// every bilinear footprint stays inside the region: the region's latent gradients live
-// in LDS (they accumulate with LDS atomics, never with global ones), and the workgroup applies
-// Adam to its region itself.  The regions of one step are distinct cells of one partition of every
+// every bilinear footprint stays inside the region: a workgroup sorts its samples by cell, sums each cell's
+// gradient in a register over the cell's samples (in a fixed order, products rounded before they are added) and
+// applies Adam to its region itself.  The regions of one step are distinct cells of one partition of every
 // grid (the partition shifts by a random offset each step), so no two workgroups touch the same
 // latent.  The MLP gradient is reduced per workgroup from per-sample records in LDS and summed over
 // workgroups in a fixed order by a second kernel, which also applies Adam to it; after a batch of
@@ -230,15 +230,19 @@ __global__ __launch_bounds__(256) void k_nm_tables(const float* mlp, float* tabl
 // launch starts with a cold L2: 2,000 cycles a hop), the MLP, its gradient.
 // - Loads that depend on nothing else go out together at the start; the cell waves load the region's Adam
 //   state, whose latents the samples read from LDS.
-// - A sample's texels come from its material's packed image: four loads on 1.6 lines (14.4 us a step) instead of
-//   six loads on six lines (18.7 us: the texel pages and lines of 65,536 samples), which maps that cannot be packed keep.
+// - A sample's texels come from its material's packed image: four loads on 1.6 lines instead of six loads on
+//   six lines (4.3 us a step less: the texel pages and lines of 65,536 samples), which maps that cannot be packed keep.
 // - The MLP runs in registers on the matrix cores (its weights were read from LDS, one wait per hidden unit).
 // - Its gradient, a product over the samples, is one matrix instruction per sample and wave from
 //   records in LDS: 256 multiply-adds in sample order for every parameter, as the scalar loops had it
 //   (three dot products of 256 LDS pairs a thread, 20,000 cycles), 29 cycles apart.
 // - Latent gradients were 32 LDS float atomics a sample (20,000 cycles): the samples are sorted by cell
 //   while their texels are on the way, and the cell waves sum them and apply Adam beside the MLP gradient.
-// 65,536 samples of 16 materials: 47 us before, 14.4 us; the MLP's update 6.2 and 5.3 us.
+//   A sample's place in its cell follows the samples' order, not the arrival of threads, and a product is rounded
+//   before it is added, as an atomic's operand is: Adam divides by the root of a second moment that may be as small as
+//   the rounding, so other last bits become other steps (two runs by atomics are 4e-5 apart after 512 steps).  The
+//   sets that give the places take 1 us of the step.
+// 65,536 samples of 16 materials: 47 us before, 15.4 us; the MLP's update 6.2 and 5.3 us.
 template <bool kExplicit>
 __global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
     constexpr uint32_t kMaxCells = kMaxR * kMaxR, kCellsPerThread = kMaxCells / 256;
@@ -306,7 +310,6 @@ __global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
             }
         }
         for (uint32_t i = tid; i < cells; i += 256) {
-            count_s[i] = 0u;
             if (!kExplicit && i < 256) {
                 lat_s[2 * i] = adam[0];
                 lat_s[2 * i + 1] = adam[1];
@@ -380,17 +383,32 @@ __global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
                 px = step_texels(T.texels, T.packed, pk, ta, tn, tm, u, v);
             }
         }
-        __syncthreads();  // counts cleared, tables written, the last chunk's records read
-        // the chunk's samples sorted by base cell while their texels and cells are on the way
+        // the chunk's samples sorted by base cell, in their order within a cell, while their texels and cells are on
+        // the way: a cell's set of samples is 256 bits (in the records' space, which is free until they are written),
+        // a sample's place in the cell its bits below the sample's own
+        uint4* const set_s = reinterpret_cast<uint4*>(rec_s);
+        for (uint32_t i = threadIdx.x; i < 2 * cells; i += kStepThreads) set_s[i] = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();  // sets cleared, tables written
         const uint32_t bin = j0 * R + i0;
-        const uint32_t rank = live ? atomicAdd(&count_s[bin], 1u) : 0u;
+        if (live) atomicOr(reinterpret_cast<uint32_t*>(set_s + 2 * bin) + (tid >> 5), 1u << (tid & 31u));
         __syncthreads();
+        uint32_t rank = 0;
+        if (live) {
+            const uint4 s0 = set_s[2 * bin], s1 = set_s[2 * bin + 1];
+            const uint32_t w[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) rank += __popc(k < (tid >> 5) ? w[k] : k == (tid >> 5) ? w[k] & ((1u << (tid & 31u)) - 1u) : 0u);
+        }
         {
             uint32_t n[kCellsPerThread] = {}, mine = 0, total;
 #pragma unroll
             for (uint32_t k = 0; k < kCellsPerThread; ++k) {
                 const uint32_t c = tid * kCellsPerThread + k;
-                if (!sampler && c < cells) n[k] = count_s[c];
+                if (!sampler && c < cells) {
+                    const uint4 s0 = set_s[2 * c], s1 = set_s[2 * c + 1];
+                    n[k] = __popc(s0.x) + __popc(s0.y) + __popc(s0.z) + __popc(s0.w) + __popc(s1.x) + __popc(s1.y) + __popc(s1.z) + __popc(s1.w);
+                    count_s[c] = n[k];
+                }
                 mine += n[k];
             }
             uint32_t at = block_exclusive_scan(mine, scan_s, total);
@@ -537,15 +555,13 @@ __global__ __launch_bounds__(kStepThreads) void k_nm_step(NmTrainLaunch T) {
                     const float w = (right ? x : 1.f - x) * (low ? y : 1.f - y);
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
-                        grad_lat[k][c] += w * d0[c];
-                        grad_lat[k][4 + c] += w * d1[c];
+                        grad_lat[k][c] += mul_rn(w, d0[c]);
+                        grad_lat[k][4 + c] += mul_rn(w, d1[c]);
                     }
                 }
             }
         }
         __syncthreads();
-        if (!sampler)
-            for (uint32_t i = tid; i < cells; i += 256) count_s[i] = 0u;
     }
     // latents of the region: gradient out (explicit mode) or Adam
     if (!sampler) {

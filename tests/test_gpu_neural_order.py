@@ -1,0 +1,69 @@
+"""Latent gradients as FP32 sums in a fixed order: a cell adds its samples' rounded products one after another, the
+samples whose footprint begins in it first, then those it is the right, lower and lower right corner of, each group in
+the samples' order.  A fused product, or an order that follows the arrival of threads, changes the last bits; Adam's
+division by the root of a small second moment turns those into whole steps, so a run would not repeat."""
+import numpy as np
+import pytest
+
+import rosy_amd
+
+pytestmark = pytest.mark.gpu
+
+
+def renderer(n_materials=2):
+    scene = rosy_amd.Scene(3, seed=2, total_triangles=20000, n_meshes=24, width=64, height=64, shadow_size=64,
+                           texture_size=64, n_materials=n_materials)
+    r = rosy_amd.Renderer(device=0)
+    r.load(scene)
+    return scene, r
+
+
+@pytest.mark.parametrize("latent,spread", [(8, 0.2), (8, 0.9), (32, 0.1)])
+def test_sum_of_rounded_products(latent, spread):
+    rng = np.random.default_rng(latent)
+    scene, r = renderer()
+    try:
+        r.neural_init(latent_size=latent, region=8, seed=5)
+        r.neural_set_params(rng.uniform(-0.8, 0.8, (2, latent, latent, 8)).astype(np.float32),
+                            rng.uniform(-0.5, 0.5, 583).astype(np.float32))
+        n, k = 64, 20  # every batch has n samples (the loss is a mean), k of them or one in the first material
+        uv = (0.05 + spread * rng.random((n, 2))).astype(np.float32)
+        target = rng.random((n, 7)).astype(np.float32)
+
+        def gradient(rows):
+            others = np.setdiff1d(np.arange(n), rows)
+            order = np.concatenate([rows, others])
+            material = np.r_[np.zeros(len(rows), np.uint32), np.ones(len(others), np.uint32)]
+            return r.neural_gradients(material, uv[order], target[order])[2][0]
+
+        # one sample's gradient at a corner is the rounded product itself
+        alone = [gradient(np.array([i])) for i in range(k)]
+        want = np.zeros_like(alone[0])
+        xy = uv[:k] * np.float32(latent) - np.float32(0.5)
+        base = np.floor(xy).astype(int)
+        for dy, dx in ((0, 0), (0, 1), (1, 0), (1, 1)):
+            for i in range(k):
+                x, y = (base[i] + (dx, dy)) % latent
+                want[y, x] += alone[i][y, x]
+        got = gradient(np.arange(k))
+        assert np.count_nonzero(want) > 8 * 8
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.abs(got - want).max()
+    finally:
+        r.close()
+        scene.close()
+
+
+@pytest.mark.parametrize("region,batch", [(2, 1024), (8, 4096), (32, 2304)])
+def test_run_repeats(region, batch):
+    runs = []
+    for _ in range(2):
+        scene, r = renderer()
+        try:
+            r.neural_init(latent_size=32, region=region, batch=batch, seed=9)
+            loss = r.neural_train(100)  # a replayed graph of steps and the remainder
+            runs.append((loss, *r.neural_params()))
+        finally:
+            r.close()
+            scene.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
