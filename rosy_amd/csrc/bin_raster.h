@@ -188,7 +188,8 @@ struct FillFragMS {  // blend view: append key | passing-sample mask << 28 to th
 
 // Edge-value products.  A record that is not wide has every coordinate difference of its edges and of its pixels
 // under 2^15, so 24-bit multiplies (full rate, with a 32-bit add; a 32-bit multiply takes four times as long) give the
-// same exact products.
+// same exact products.  k_raster<32, 4> at 1600 x 900: 70 and 66 us; one sample, a 2560 x 1440 frame with four cascades:
+// 52 and 50 us.
 template <typename EdgeT>
 __device__ inline EdgeT edge_mul(int32_t a, int32_t b) {
     if constexpr (sizeof(EdgeT) == 4) return __mul24(a, b);
@@ -277,10 +278,11 @@ __device__ inline void raster_row_ms(const TriRec& r, uint32_t meta, int ox, int
 
 // LDS of one work item's records.  Tasks are rows, and with 4 samples row segments of eight pixels: a wave takes as
 // long as its longest task, and a pixel costs four times as much there (k_raster<32, 4> with whole rows and with
-// segments: 79 and 68 us at 1600 x 900; with one sample the segments' own cost outweighs it: 55 and 60 us for the
+// segments: 76 and 67 us at 1600 x 900; with one sample the segments' own cost outweighs it, by a tenth in the
 // views of a 2560 x 1440 frame with four cascades).  A task finds its record by a bit per task (set where a record's
-// tasks begin) and the count of records that began before the 64 tasks of its word; a table of one byte a task took
-// a serial store loop per record and twice the space (58 us for the same views).
+// tasks begin) and the count of records that began before the 64 tasks of its word: half the space of a table of one
+// byte a task and no store loop per record, for k_blend_collect's workgroups a CU and the many tasks of segments (one
+// sample alone gains nothing: 89 us by the table and 90 in the 2M-triangle frame, 202 and 200 with bins of 8 pixels).
 template <int T, int N>
 struct RasterLds {
     static constexpr int kSeg = N == 4 ? 8 : T, kSegs = T / kSeg;

@@ -984,8 +984,7 @@ __device__ inline float4 blend_over(float4 dst, float4 f) {
 }
 
 template <int T, int N>
-__global__ __launch_bounds__(256) void k_blend_resolve(const BlendLaunch B, const ShadeLaunch L) {
-    if (B.report && blockIdx.x + 1u == gridDim.x) report_counters(B.report, B.counters, B.n_views, B.totals);
+__device__ __forceinline__ void blend_pixel(const BlendLaunch& B, const ShadeLaunch& L) {
     uint32_t vi = 0;
     while (vi + 1 < L.n_views && L.views[vi + 1].block_base <= blockIdx.x) ++vi;
     const ShadeView& SV = L.views[vi];
@@ -1026,6 +1025,13 @@ __global__ __launch_bounds__(256) void k_blend_resolve(const BlendLaunch B, cons
         }
         SV.color[o] = c;
     }
+}
+
+template <int T, int N>
+__global__ __launch_bounds__(256) void k_blend_resolve(const BlendLaunch B, const ShadeLaunch L) {
+    blend_pixel<T, N>(B, L);
+    // (last: see k_raster; 16 us with the report first, 13.8 this way)
+    if (B.report && blockIdx.x + 1u == gridDim.x) report_counters(B.report, B.counters, B.n_views, B.totals);
 }
 
 hipError_t launch_blend_fragments(const BlendLaunch& b, const ShadeLaunch& l, hipStream_t s) {
