@@ -285,7 +285,8 @@ rsy_result rsy_set_geometry(rsy_ctx* ctx, const rsy_position* vertices, uint64_t
                             const rsy_mesh_range* meshes, uint32_t n_meshes);
 
 /* Materials, samplers and decoded texture images.  Replaces the image, sampler and material
- * upload in set_asset (Graphics.cpp:3590-4160). */
+ * upload in set_asset (Graphics.cpp:3590-4160).  Arguments are checked before anything changes; a
+ * call that fails after that, for want of memory, leaves the context without materials. */
 rsy_result rsy_set_materials(rsy_ctx* ctx, const rsy_gpu_material* materials, uint32_t n_materials,
                              const rsy_texture_desc* textures, uint32_t n_textures,
                              const rsy_sampler* samplers, uint32_t n_samplers);

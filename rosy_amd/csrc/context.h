@@ -49,6 +49,7 @@ struct DevBuf {
         const size_t want = std::max<size_t>(bytes, 256);
         hipError_t e = hipMalloc(&p, want);
         if (e != hipSuccess) {
+            (void)hipGetLastError();  // (else the next launch would report it)
             p = nullptr;
             return e;
         }
@@ -217,8 +218,8 @@ struct rsy_ctx {
     std::vector<rsy::PackGPU> h_packs;  // per material
     std::vector<uint8_t> tex_opaque;  // four-channel texture whose alpha is 255 everywhere
     rsy::DevBuf tex_staging;          // BC7 blocks on their way to the decoder
-    rsy::DevBuf tex_jobs, tex_flags;  // the upload kernels' images and alpha-test results
-    rsy::DevBuf packs, packed, pack_jobs;  // packed materials: per material, their texels, the upload's jobs
+    rsy::DevBuf tex_jobs;             // the upload kernels' images, alpha-test results and images to pack
+    rsy::DevBuf packs, packed;        // packed materials: per material, their texels
     rsy::DevBuf mip_tables;           // byte values of the mip filter (made at the first built chain)
     bool any_mips = false;            // some texture has more than one level (LOD sampling)
     // draw lists: 0 = shadow (all), 1 = opaque (!blended), 2 = blended (the blended pass)
