@@ -290,6 +290,10 @@ rsy_result rsy_set_geometry(rsy_ctx* ctx, const rsy_position* vertices, uint64_t
 rsy_result rsy_set_materials(rsy_ctx* ctx, const rsy_gpu_material* materials, uint32_t n_materials,
                              const rsy_texture_desc* textures, uint32_t n_textures,
                              const rsy_sampler* samplers, uint32_t n_samplers);
+/* How many materials are sampled as one packed image (a second copy of their maps, made by
+ * rsy_set_materials for those whose maps are alike, while it takes at most twice the texels' memory
+ * and a quarter of what is free), and the bytes of those images.  No counterpart in the reference. */
+rsy_result rsy_get_packed_materials(rsy_ctx* ctx, uint32_t* n_packed, uint64_t* bytes);
 
 /* Object records and surfaces; builds the shadow (all), opaque (!blended) and blended lists in
  * the order given.  Replaces graphics_device::set_graphic_objects (Graphics.cpp:4691-4921). */
@@ -350,6 +354,7 @@ rsy_result rsy_get_device_outputs(rsy_ctx* ctx, uint32_t view, const void** vis,
                                       and give a new layout's first frame 64 raster workgroups, too
                                       few for its work items, so that it is re-run with a grid that
                                       fits */
+#define RSY_DEBUG_MIN_PACK 8u      /* let packed materials take 16 KiB (at the next rsy_set_materials) */
 rsy_result rsy_set_debug_flags(rsy_ctx* ctx, uint32_t flags);
 
 /* The output stage of the last shaded frame for one camera view (Graphics.cpp:1908, 5835-5880):

@@ -178,6 +178,12 @@ class Renderer:
     def synchronize(self):
         self._c(lib().rsy_synchronize(self.ctx), "rsy_synchronize")
 
+    def packed_materials(self):
+        """(materials sampled as one packed image, bytes of those images)."""
+        n, b = C.c_uint32(), C.c_uint64()
+        self._c(lib().rsy_get_packed_materials(self.ctx, C.byref(n), C.byref(b)), "rsy_get_packed_materials")
+        return n.value, b.value
+
     def set_debug_flags(self, flags):
         self._c(lib().rsy_set_debug_flags(self.ctx, flags), "rsy_set_debug_flags")
 

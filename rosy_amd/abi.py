@@ -23,7 +23,7 @@ RSY_ABSENT = 0xFFFFFFFF
 RSY_ABI_VERSION = 1
 SHADE_NONE, SHADE_PLAIN, SHADE_NEURAL = 0, 1, 2
 PCF_REFERENCE_5TAP, PCF_GRID_3X3 = 0, 1
-DEBUG_SHADOW_FACTOR, DEBUG_STAGE_TIMING, DEBUG_MIN_CAPACITY = 1, 2, 4
+DEBUG_SHADOW_FACTOR, DEBUG_STAGE_TIMING, DEBUG_MIN_CAPACITY, DEBUG_MIN_PACK = 1, 2, 4, 8
 TEX_RGBA8_SRGB, TEX_RGBA8_UNORM, TEX_RG8_UNORM, TEX_RG8_SRGB, TEX_BC7_SRGB, TEX_BC7_UNORM = 0, 1, 2, 3, 4, 5
 MIPS_BUILD = 0xFFFFFFFF
 
@@ -240,6 +240,7 @@ PROTOTYPES = [
                                    C.POINTER(MeshRange), C.c_uint32]),
     ("rsy_set_materials", C.c_int, [C.c_void_p, C.POINTER(GpuMaterial), C.c_uint32, C.POINTER(TextureDesc),
                                     C.c_uint32, C.POINTER(Sampler), C.c_uint32]),
+    ("rsy_get_packed_materials", C.c_int, [C.c_void_p, C.POINTER(C.c_uint32), C.POINTER(C.c_uint64)]),
     ("rsy_set_graphic_objects", C.c_int, [C.c_void_p, C.POINTER(ObjectRecord), C.c_uint32, C.POINTER(Draw),
                                           C.c_uint32]),
     ("rsy_update_graphic_objects", C.c_int, [C.c_void_p, C.c_uint64, C.POINTER(ObjectRecord), C.c_uint32]),

@@ -1040,9 +1040,10 @@ namespace {
 // with the same addressing.  Others (a map missing, a four-channel normal map, sizes that differ, nearest filtering)
 // keep their maps: one packed sample needs one set of coordinates (map by map, with four-channel normals, k_shade
 // takes 57 us at 1920 x 1080 and 61 with chains, k_shade_ms 89 at 1366 x 768).  Materials with the same maps share one
-// image.  Returns the bytes of the packed texels.
+// image, but a map that several of them combine with others is copied into each: materials whose image would take the
+// copies past `budget` bytes keep their maps, too.  Returns the bytes of the packed texels.
 uint64_t plan_packs(const rsy_gpu_material* materials, uint32_t n_materials, const std::vector<TexGPU>& table,
-                    const rsy_sampler* samplers, uint32_t n_samplers, std::vector<PackGPU>& packs,
+                    const rsy_sampler* samplers, uint32_t n_samplers, uint64_t budget, std::vector<PackGPU>& packs,
                     std::vector<PackJob>& jobs, uint32_t& max_tiles) {
     packs.assign(n_materials, PackGPU{});
     std::map<std::array<uint32_t, 3>, uint64_t> made;  // maps -> offset
@@ -1073,6 +1074,7 @@ uint64_t plan_packs(const rsy_gpu_material* materials, uint32_t n_materials, con
         if (at == made.end()) {
             uint32_t tiles = 0;
             for (uint32_t l = 0; l < c.levels; ++l) tiles += pack_tiles(c.width, c.height, l);
+            if (bytes + uint64_t(tiles) * 128 > budget) continue;
             at = made.emplace(key, bytes).first;
             jobs.push_back({c, n, r, bytes});
             max_tiles = std::max(max_tiles, tiles);
@@ -1082,6 +1084,19 @@ uint64_t plan_packs(const rsy_gpu_material* materials, uint32_t n_materials, con
                     mode | (r.srgb ? kPackMrSrgb : 0u)};
     }
     return bytes;
+}
+
+// What the packed images of `pool` bytes of texels may take.  A map that is in one material only is copied once
+// and at its own size, so twice the pool leaves room for shared ones; large copies stay within a quarter of the
+// memory that is free, which the frame's and the decoder's buffers still need.  (The question takes the runtime
+// some microseconds, more than copies that small could matter.)
+uint64_t pack_budget(const rsy_ctx* c, uint64_t pool) {
+    if (c->debug_flags & RSY_DEBUG_MIN_PACK) return 16u << 10;
+    uint64_t budget = 2 * pool;
+    size_t free_bytes = 0, total = 0;
+    if (budget > (64u << 20) && hipMemGetInfo(&free_bytes, &total) == hipSuccess)
+        budget = std::min<uint64_t>(budget, (free_bytes + c->packed.cap) / 4);
+    return budget;
 }
 
 // No materials, textures or samplers, and no decoder of them.
@@ -1094,6 +1109,7 @@ void forget_materials(rsy_ctx* c) {
     c->h_packs.clear();
     c->h_samplers.clear();
     c->any_mips = false;
+    c->pack_bytes = 0;
     destroy_neural(c->neural);
     c->neural = nullptr;
     invalidate_graph(c);
@@ -1155,6 +1171,7 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     // from here the previous materials are gone: a call that fails leaves the context without any
     forget_materials(c);
     // every allocation before the first copy
+    if (pool > c->texels.cap) c->packed.release();  // (the texels come first)
     HIP_TRY(c, c->materials.ensure(std::max<size_t>(1, n_materials) * sizeof(rsy_gpu_material)), "allocate materials");
     HIP_TRY(c, c->tex_table.ensure(std::max<size_t>(1, n_textures) * sizeof(TexGPU)), "allocate textures");
     HIP_TRY(c, c->texels.ensure(std::max<uint64_t>(256, pool)), "allocate texels");
@@ -1163,12 +1180,13 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     HIP_TRY(c, c->packs.ensure(std::max<size_t>(1, n_materials) * sizeof(PackGPU)), "allocate packed materials");
     std::vector<PackJob> pack_jobs;
     uint32_t pack_tiles_max = 0;
-    uint64_t pack_bytes = plan_packs(materials, n_materials, table, samplers, n_samplers, packs, pack_jobs, pack_tiles_max);
+    uint64_t pack_bytes = plan_packs(materials, n_materials, table, samplers, n_samplers, pack_budget(c, pool), packs, pack_jobs, pack_tiles_max);
     if (pack_bytes && c->packed.ensure(pack_bytes) != hipSuccess) {
         for (PackGPU& k : packs) k.levels = 0;  // no room for a second copy of the texels: the maps are sampled one by one
         pack_jobs.clear();
         pack_bytes = 0;
     }
+    if (!pack_bytes) c->packed.release();
     // the upload kernels' tables in one block: images, alpha-test results, images to pack
     const size_t flags_at = (jobs.size() * sizeof(MipJob) + 255) & ~size_t(255);
     const size_t packs_at = flags_at + ((size_t(n_textures) * 4 + 255) & ~size_t(255));
@@ -1243,6 +1261,7 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     c->h_materials.assign(materials, materials + n_materials);
     c->h_tex_table = table;
     c->h_packs = packs;
+    c->pack_bytes = pack_bytes;
     c->h_samplers.assign(samplers, samplers + n_samplers);
     // the draws' sampler flags follow the materials: refreshed in place, so that the allocation-free
     // render path keeps working after a material change
@@ -1259,6 +1278,14 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
         c->any_mips |= table[t].levels > 1;
         if (table[t].channels == 4) c->tex_opaque[t] = opaque[t] ? 1 : 0;
     }
+    return RSY_OK;
+}
+
+rsy_result rsy_get_packed_materials(rsy_ctx* c, uint32_t* n_packed, uint64_t* bytes) {
+    if (!c || !n_packed || !bytes) return RSY_INVALID_ARGUMENT;
+    *n_packed = 0;
+    for (const PackGPU& k : c->h_packs) *n_packed += k.levels != 0;
+    *bytes = c->pack_bytes;
     return RSY_OK;
 }
 

@@ -220,6 +220,7 @@ struct rsy_ctx {
     rsy::DevBuf tex_staging;          // BC7 blocks on their way to the decoder
     rsy::DevBuf tex_jobs;             // the upload kernels' images, alpha-test results and images to pack
     rsy::DevBuf packs, packed;        // packed materials: per material, their texels
+    uint64_t pack_bytes = 0;          // of `packed` in use
     rsy::DevBuf mip_tables;           // byte values of the mip filter (made at the first built chain)
     bool any_mips = false;            // some texture has more than one level (LOD sampling)
     // draw lists: 0 = shadow (all), 1 = opaque (!blended), 2 = blended (the blended pass)
