@@ -211,14 +211,20 @@ __device__ inline void nm_mlp_wave(const NmWeights* __restrict__ W, const float 
     h8 q1h = __builtin_bit_cast(h8, ph), q1l = __builtin_bit_cast(h8, pl);
     nm_swap32(q0h, q1h);  // q0: tile 0's operand (lower lanes the first half, upper lanes the second), q1: tile 1's
     nm_swap32(q0l, q1l);
-    // both layers' scales are applied to the outputs: relu(s1 x) = s1 relu(x) for s1 > 0
-    const float s12 = W->scale[0] * W->scale[1];
+    // layer 1's scale goes on its accumulator (1 in the FP16 form): stored codes are up to 1.75 whatever the weights,
+    // and times features of a few thousand they would leave the halves' range (k_nm_eval with FP8 weights, 32 materials of
+    // 1024^2 texels: 452 us, 430 with both scales on the outputs; frames the same)
+    const bool scaled = W->fp8 != 0u;
+    const float s1 = W->scale[0], s2 = W->scale[1];
     uint32_t res[2][4];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         f32x16 acc = {};
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, t == 0 ? q0h : q1h, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, t == 0 ? q0l : q1l, acc, 0, 0, 0);
+        if (scaled)  // uniform
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] *= s1;
         f32x16 acc2 = {};
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -242,7 +248,7 @@ __device__ inline void nm_mlp_wave(const NmWeights* __restrict__ W, const float 
         if (r < 3) out[4 + r] = __uint_as_float(res[1][r]);
     }
 #pragma unroll
-    for (int c = 0; c < kNmOut; ++c) out[c] = __builtin_amdgcn_fmed3f(fmaf(out[c], s12, W->b2[c]), 0.f, 1.f);
+    for (int c = 0; c < kNmOut; ++c) out[c] = __builtin_amdgcn_fmed3f(fmaf(out[c], s2, W->b2[c]), 0.f, 1.f);
 }
 
 }  // namespace rsy
