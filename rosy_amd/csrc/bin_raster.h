@@ -58,9 +58,8 @@ __device__ inline uint32_t fbits(float f) { return __float_as_uint(f); }
 // kernel that runs after they are final: the two small copies this replaces were blit kernels of 4.5 us.
 __device__ inline void report_counters(uint32_t* report, const uint32_t* counters, uint32_t n_views, const uint32_t* totals) {
     const uint32_t n = n_views * kCtrPerView;
-    if (threadIdx.x < n + 4u)
-        __hip_atomic_store(report + threadIdx.x, threadIdx.x < n ? counters[threadIdx.x] : totals[threadIdx.x - n],
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (uint32_t i = threadIdx.x; i < n + 4u; i += blockDim.x)
+        __hip_atomic_store(report + i, i < n ? counters[i] : totals[i - n], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 constexpr uint32_t kItemRecs = 256;   // records per raster work item (one per thread)
