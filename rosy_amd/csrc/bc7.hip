@@ -323,11 +323,6 @@ __global__ __launch_bounds__(256) void k_pack(const PackJob* jobs, const uint8_t
     }
 }
 
-__global__ void k_set_flags(uint32_t* flags, uint32_t n) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) flags[i] = 1u;
-}
-
 }  // namespace
 
 hipError_t launch_mip_tables(double* tables, hipStream_t s) {
@@ -348,8 +343,6 @@ hipError_t launch_build_mips(const MipJob* jobs, uint32_t n_jobs, uint32_t max_w
 }
 
 hipError_t launch_alpha_test(const MipJob* jobs, uint32_t n_jobs, const uint8_t* texels, uint32_t* flags, hipStream_t s) {
-    if (n_jobs == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_set_flags, dim3((n_jobs + 255) / 256), dim3(256), 0, s, flags, n_jobs);
     for (uint32_t first = 0; first < n_jobs; first += 65535u)
         hipLaunchKernelGGL(k_alpha_test, dim3(256, min(n_jobs - first, 65535u)), dim3(256), 0, s, jobs + first, texels,
                            flags + first);

@@ -695,14 +695,14 @@ rsy_result enqueue_frame(rsy_ctx* c, const Layout& L, const FrameMem& m, bool ca
         sh.indices = g.indices;
         sh.vertices = c->vertices.p;
         sh.objects = g.objects;
-        sh.materials = c->materials.p;
+        sh.materials = c->tables.materials;
         sh.n_materials = c->n_materials;
-        sh.textures = c->tex_table.as<TexGPU>();
+        sh.textures = c->tables.textures;
         sh.n_textures = c->n_textures;
         sh.texels = c->texels.as<uint8_t>();
-        sh.packs = c->packs.as<PackGPU>();
+        sh.packs = c->tables.packs;
         sh.packed = c->packed.as<uint8_t>();
-        sh.samplers = c->samplers.p;
+        sh.samplers = c->tables.samplers;
         sh.n_samplers = c->n_samplers;
         std::memcpy(sh.clear_color, c->rs.clear_color, sizeof(sh.clear_color));
         sh.srgb_lut = c->srgb_lut.as<float>();
@@ -1102,6 +1102,7 @@ uint64_t pack_budget(const rsy_ctx* c, uint64_t pool) {
 // No materials, textures or samplers, and no decoder of them.
 void forget_materials(rsy_ctx* c) {
     c->n_materials = c->n_textures = c->n_samplers = 0;
+    c->tables = MaterialTables{};
     c->tex_channels.clear();
     c->tex_opaque.clear();
     c->h_materials.clear();
@@ -1172,12 +1173,8 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     forget_materials(c);
     // every allocation before the first copy
     if (pool > c->texels.cap) c->packed.release();  // (the texels come first)
-    HIP_TRY(c, c->materials.ensure(std::max<size_t>(1, n_materials) * sizeof(rsy_gpu_material)), "allocate materials");
-    HIP_TRY(c, c->tex_table.ensure(std::max<size_t>(1, n_textures) * sizeof(TexGPU)), "allocate textures");
     HIP_TRY(c, c->texels.ensure(std::max<uint64_t>(256, pool)), "allocate texels");
-    HIP_TRY(c, c->samplers.ensure(std::max<size_t>(1, n_samplers) * sizeof(rsy_sampler)), "allocate samplers");
     if (staging) HIP_TRY(c, c->tex_staging.ensure(staging), "allocate texture staging");
-    HIP_TRY(c, c->packs.ensure(std::max<size_t>(1, n_materials) * sizeof(PackGPU)), "allocate packed materials");
     std::vector<PackJob> pack_jobs;
     uint32_t pack_tiles_max = 0;
     uint64_t pack_bytes = plan_packs(materials, n_materials, table, samplers, n_samplers, pack_budget(c, pool), packs, pack_jobs, pack_tiles_max);
@@ -1187,13 +1184,27 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
         pack_bytes = 0;
     }
     if (!pack_bytes) c->packed.release();
-    // the upload kernels' tables in one block: images, alpha-test results, images to pack
-    const size_t flags_at = (jobs.size() * sizeof(MipJob) + 255) & ~size_t(255);
-    const size_t packs_at = flags_at + ((size_t(n_textures) * 4 + 255) & ~size_t(255));
-    HIP_TRY(c, c->tex_jobs.ensure(packs_at + pack_jobs.size() * sizeof(PackJob)), "allocate texture jobs");
-    MipJob* const mip_d = c->tex_jobs.as<MipJob>();
-    uint32_t* const flags_d = reinterpret_cast<uint32_t*>(c->tex_jobs.as<uint8_t>() + flags_at);
-    PackJob* const pack_d = reinterpret_cast<PackJob*>(c->tex_jobs.as<uint8_t>() + packs_at);
+    const std::vector<uint32_t> ones(n_textures, 1u);
+    std::vector<uint8_t> image;  // of the tables
+    const auto put = [&](const auto* from, size_t n) {
+        const size_t at = image.size(), bytes = n * sizeof(*from);
+        image.resize(at + std::max<size_t>(256, (bytes + 255) & ~size_t(255)));
+        if (bytes) std::memcpy(image.data() + at, from, bytes);
+        return at;
+    };
+    const size_t at[7] = {put(materials, n_materials), put(packs.data(), packs.size()), put(table.data(), table.size()),
+                          put(samplers, n_samplers), put(jobs.data(), jobs.size()), put(ones.data(), ones.size()),
+                          put(pack_jobs.data(), pack_jobs.size())};
+    HIP_TRY(c, c->tables_mem.ensure(image.size()), "allocate material tables");
+    uint8_t* const block = c->tables_mem.as<uint8_t>();
+    MaterialTables& T = c->tables;
+    T.materials = reinterpret_cast<rsy_gpu_material*>(block + at[0]);
+    T.packs = reinterpret_cast<PackGPU*>(block + at[1]);
+    T.textures = reinterpret_cast<TexGPU*>(block + at[2]);
+    T.samplers = reinterpret_cast<rsy_sampler*>(block + at[3]);
+    T.mip_jobs = reinterpret_cast<MipJob*>(block + at[4]);
+    T.opaque = reinterpret_cast<uint32_t*>(block + at[5]);
+    T.pack_jobs = reinterpret_cast<PackJob*>(block + at[6]);
     const bool make_tables = max_levels && !c->mip_tables.p;
     if (make_tables) HIP_TRY(c, c->mip_tables.ensure(512 * sizeof(double)), "allocate mip tables");
 
@@ -1204,16 +1215,7 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
         if (e != hipSuccess) c->mip_tables.release();
         HIP_TRY(c, e, "mip tables");
     }
-    if (n_materials) {
-        HIP_TRY(c, hipMemcpy(c->materials.p, materials, n_materials * sizeof(rsy_gpu_material), hipMemcpyHostToDevice), "upload materials");
-        HIP_TRY(c, hipMemcpyAsync(c->packs.p, packs.data(), packs.size() * sizeof(PackGPU), hipMemcpyHostToDevice, c->stream),
-                "upload packed materials");
-    }
-    if (n_textures) {
-        HIP_TRY(c, hipMemcpy(c->tex_table.p, table.data(), n_textures * sizeof(TexGPU), hipMemcpyHostToDevice), "upload textures");
-        HIP_TRY(c, hipMemcpyAsync(mip_d, jobs.data(), jobs.size() * sizeof(MipJob), hipMemcpyHostToDevice, c->stream),
-                "upload texture jobs");
-    }
+    HIP_TRY(c, hipMemcpyAsync(block, image.data(), image.size(), hipMemcpyHostToDevice, c->stream), "upload material tables");
     // the given levels first (a BC7 image is decoded while the next image is copied), then every built chain and
     // the alpha test of every image, in a few launches over all of them
     uint64_t staged = 0;  // every BC7 image's blocks go to their own part of the staging buffer
@@ -1239,20 +1241,16 @@ rsy_result rsy_set_materials(rsy_ctx* c, const rsy_gpu_material* materials, uint
     }
     if (n_textures) {
         if (max_levels)
-            HIP_TRY(c, launch_build_mips(mip_d + n_textures, uint32_t(jobs.size() - n_textures), max_w, max_h, max_levels,
+            HIP_TRY(c, launch_build_mips(T.mip_jobs + n_textures, uint32_t(jobs.size() - n_textures), max_w, max_h, max_levels,
                                          c->texels.as<uint8_t>(), c->mip_tables.as<double>(), c->stream), "build mip levels");
-        HIP_TRY(c, launch_alpha_test(mip_d, n_textures, c->texels.as<uint8_t>(), flags_d, c->stream), "alpha test");
-        HIP_TRY(c, hipMemcpyAsync(opaque.data(), flags_d, size_t(n_textures) * 4, hipMemcpyDeviceToHost, c->stream),
+        HIP_TRY(c, launch_alpha_test(T.mip_jobs, n_textures, c->texels.as<uint8_t>(), T.opaque, c->stream), "alpha test");
+        HIP_TRY(c, hipMemcpyAsync(opaque.data(), T.opaque, size_t(n_textures) * 4, hipMemcpyDeviceToHost, c->stream),
                 "read alpha test");
     }
-    if (!pack_jobs.empty()) {
-        HIP_TRY(c, hipMemcpyAsync(pack_d, pack_jobs.data(), pack_jobs.size() * sizeof(PackJob), hipMemcpyHostToDevice,
-                                  c->stream), "upload pack jobs");
-        HIP_TRY(c, launch_pack(pack_d, uint32_t(pack_jobs.size()), pack_tiles_max, c->texels.as<uint8_t>(),
+    if (!pack_jobs.empty())
+        HIP_TRY(c, launch_pack(T.pack_jobs, uint32_t(pack_jobs.size()), pack_tiles_max, c->texels.as<uint8_t>(),
                                c->packed.as<uint8_t>(), c->stream), "pack materials");
-    }
     HIP_TRY(c, hipStreamSynchronize(c->stream), "synchronize");
-    if (n_samplers) HIP_TRY(c, hipMemcpy(c->samplers.p, samplers, n_samplers * sizeof(rsy_sampler), hipMemcpyHostToDevice), "upload samplers");
     c->n_materials = n_materials;
     c->n_textures = n_textures;
     c->n_samplers = n_samplers;

@@ -86,6 +86,18 @@ struct PinnedBuf {
     }
 };
 
+// The tables of the materials and of their upload, device addresses in one block that one copy fills (a small
+// copy takes 10 us of the host, an allocation as much).
+struct MaterialTables {
+    rsy_gpu_material* materials = nullptr;
+    PackGPU* packs = nullptr;     // per material
+    TexGPU* textures = nullptr;
+    rsy_sampler* samplers = nullptr;
+    MipJob* mip_jobs = nullptr;   // every image, then the ones whose chains are built
+    uint32_t* opaque = nullptr;   // the alpha test's results, 1 at first
+    PackJob* pack_jobs = nullptr;
+};
+
 struct FrameViewDesc {
     bool shadow;
     uint32_t width, height;
@@ -209,7 +221,9 @@ struct rsy_ctx {
     std::vector<rsy_draw> surfaces;
     bool has_objects = false;
     // materials
-    rsy::DevBuf materials, tex_table, texels, samplers, srgb_lut;
+    rsy::DevBuf texels, srgb_lut;
+    rsy::MaterialTables tables;
+    rsy::DevBuf tables_mem;           // all of them
     uint32_t n_materials = 0, n_textures = 0, n_samplers = 0;
     std::vector<uint32_t> tex_channels;
     std::vector<rsy_gpu_material> h_materials;
@@ -218,8 +232,7 @@ struct rsy_ctx {
     std::vector<rsy::PackGPU> h_packs;  // per material
     std::vector<uint8_t> tex_opaque;  // four-channel texture whose alpha is 255 everywhere
     rsy::DevBuf tex_staging;          // BC7 blocks on their way to the decoder
-    rsy::DevBuf tex_jobs;             // the upload kernels' images, alpha-test results and images to pack
-    rsy::DevBuf packs, packed;        // packed materials: per material, their texels
+    rsy::DevBuf packed;               // the texels of packed materials
     uint64_t pack_bytes = 0;          // of `packed` in use
     rsy::DevBuf mip_tables;           // byte values of the mip filter (made at the first built chain)
     bool any_mips = false;            // some texture has more than one level (LOD sampling)

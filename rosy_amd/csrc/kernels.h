@@ -271,7 +271,7 @@ struct NmPointLaunch {
 };
 
 // texture upload: the BC7 blocks of an image's levels into RGBA8 texels; the byte tables of the mip filter; the
-// chains of the images in `jobs`, each from its level 0; flags[i] = 1 when image i is opaque (four channels)
+// chains of the images in `jobs`, each from its level 0; flags[i], 1 before, becomes 0 when image i has four channels and is not opaque
 hipError_t launch_bc7_decode(const void* blocks, uint32_t width, uint32_t height, uint32_t levels, uint32_t* rgba,
                              hipStream_t s);
 hipError_t launch_mip_tables(double* tables, hipStream_t s);

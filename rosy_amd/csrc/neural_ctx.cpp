@@ -28,7 +28,7 @@ struct NeuralState {
     std::vector<uint32_t> block_base;  // evaluation tiles per slot (prefix, n_slots + 1)
     uint32_t max_tiles = 0;            // of the largest slot
     bool any_same = false, any_other = false;  // some slot's maps share one extent / differ in size
-    DevBuf slots_d, maps_d, packs_d, slot_of_d, active_d, block_base_d;
+    DevBuf slots_d, maps_d, slot_of_d, active_d, block_base_d;
     DevBuf lat, lat_m, lat_v, mlp, mlp_m, mlp_v, tables, partial, step_d, loss_d, lat16, weights_d, eval_partial, eval_sum;
     DevBuf tmp[5];
     uint32_t n_wg = 0, spw = 0;
@@ -133,10 +133,11 @@ NmTrainLaunch train_args(rsy_ctx* c, NeuralState* n) {
     T.tables = n->tables.as<float>();
     T.partial = n->partial.as<float>();
     T.step = n->step_d.as<uint32_t>();
-    T.maps = n->maps_d.as<TexGPU>();
+    T.maps = n->maps_d.as<TexGPU>();  // the packed images' records follow
+    static_assert(sizeof(TexGPU) % alignof(PackGPU) == 0, "records in one block");
     T.n_slots = uint32_t(n->slots.size());
     T.texels = c->texels.as<uint8_t>();
-    T.packs = n->packs_d.as<PackGPU>();
+    T.packs = reinterpret_cast<const PackGPU*>(T.maps + 3 * n->slots.size());
     T.packed = c->packed.as<uint8_t>();
     T.srgb_lut = c->srgb_lut.as<float>();
     T.L = n->L;
@@ -241,8 +242,7 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     HIP_TRY(c, hipEventCreate(&n->ev0), "event");
     HIP_TRY(c, hipEventCreate(&n->ev1), "event");
     HIP_TRY(c, n->slots_d.ensure(std::max<size_t>(1, ns) * sizeof(NmSlot)), "allocate decoder");
-    HIP_TRY(c, n->maps_d.ensure(std::max<size_t>(1, ns) * 3 * sizeof(TexGPU)), "allocate decoder");
-    HIP_TRY(c, n->packs_d.ensure(std::max<size_t>(1, ns) * sizeof(PackGPU)), "allocate decoder");
+    HIP_TRY(c, n->maps_d.ensure(std::max<size_t>(1, ns) * (3 * sizeof(TexGPU) + sizeof(PackGPU))), "allocate decoder");
     HIP_TRY(c, n->slot_of_d.ensure(std::max<size_t>(1, nm) * 4), "allocate decoder");
     HIP_TRY(c, n->active_d.ensure(std::max<size_t>(1, nm) * 4), "allocate decoder");
     HIP_TRY(c, n->block_base_d.ensure((ns + 1) * 4), "allocate decoder");
@@ -262,14 +262,18 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     HIP_TRY(c, n->eval_partial.ensure(size_t(std::max<uint32_t>(1, n->block_base[ns])) * 4), "allocate decoder");
     HIP_TRY(c, n->eval_sum.ensure(std::max<size_t>(1, ns) * 8), "allocate decoder");
     if (ns) {
-        std::vector<TexGPU> maps;
-        std::vector<PackGPU> packs;
-        for (const NmSlot& sl : n->slots) packs.push_back(c->h_packs[sl.material]);
-        HIP_TRY(c, hipMemcpy(n->packs_d.p, packs.data(), packs.size() * sizeof(PackGPU), hipMemcpyHostToDevice), "upload");
-        for (const NmSlot& sl : n->slots)
-            for (uint32_t k : {sl.albedo, sl.normal, sl.mr}) maps.push_back(c->h_tex_table[k]);
+        std::vector<uint8_t> maps(ns * (3 * sizeof(TexGPU) + sizeof(PackGPU)));
+        uint8_t *map = maps.data(), *pack = map + ns * 3 * sizeof(TexGPU);
+        for (const NmSlot& sl : n->slots) {
+            for (uint32_t k : {sl.albedo, sl.normal, sl.mr}) {
+                std::memcpy(map, &c->h_tex_table[k], sizeof(TexGPU));
+                map += sizeof(TexGPU);
+            }
+            std::memcpy(pack, &c->h_packs[sl.material], sizeof(PackGPU));
+            pack += sizeof(PackGPU);
+        }
         HIP_TRY(c, hipMemcpy(n->slots_d.p, n->slots.data(), ns * sizeof(NmSlot), hipMemcpyHostToDevice), "upload");
-        HIP_TRY(c, hipMemcpy(n->maps_d.p, maps.data(), maps.size() * sizeof(TexGPU), hipMemcpyHostToDevice), "upload");
+        HIP_TRY(c, hipMemcpy(n->maps_d.p, maps.data(), maps.size(), hipMemcpyHostToDevice), "upload");
     }
     if (nm) {
         HIP_TRY(c, hipMemcpy(n->slot_of_d.p, n->slot_of.data(), nm * 4, hipMemcpyHostToDevice), "upload");
@@ -291,7 +295,7 @@ rsy_result rsy_neural_init(rsy_ctx* c, const rsy_neural_config* cfg) {
     I.random = cfg->init == RSY_NEURAL_INIT_RANDOM ? 1u : 0u;
     I.seed = cfg->seed;
     I.slots = n->slots_d.p;
-    I.textures = c->tex_table.as<TexGPU>();
+    I.textures = c->tables.textures;
     I.texels = c->texels.as<uint8_t>();
     I.srgb_lut = c->srgb_lut.as<float>();
     HIP_TRY(c, launch_nm_init(I, s), "initialise latents");
@@ -365,7 +369,7 @@ rsy_result rsy_neural_evaluate(rsy_ctx* c, float* psnr, uint32_t n_materials) {
     E.slots = n->slots_d.p;
     E.n_slots = ns;
     E.block_base = n->block_base_d.as<uint32_t>();
-    E.textures = c->tex_table.as<TexGPU>();
+    E.textures = c->tables.textures;
     E.texels = c->texels.as<uint8_t>();
     E.srgb_lut = c->srgb_lut.as<float>();
     E.partial = n->eval_partial.as<float>();
@@ -568,7 +572,7 @@ rsy_result rsy_neural_decode(rsy_ctx* c, const uint32_t* material, const float* 
     P.uv = n->tmp[0].as<float>();
     P.n = n_pts;
     P.targets = targets ? 1u : 0u;
-    P.textures = c->tex_table.as<TexGPU>();
+    P.textures = c->tables.textures;
     P.texels = c->texels.as<uint8_t>();
     P.srgb_lut = c->srgb_lut.as<float>();
     P.out = n->tmp[1].as<float>();
