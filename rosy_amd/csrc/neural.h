@@ -51,7 +51,7 @@ struct NmWeights {
     float b2[8];
     float scale[2];
     uint32_t fp8;
-    uint32_t pad;
+    uint32_t first;  // two halves: 2^e, which layer 1's widened codes are multiplied by, and 2^-e (nm_first_scale)
 };
 static_assert(sizeof(NmWeights) == kNmWeightsBytes, "NmWeights layout");
 
@@ -176,6 +176,19 @@ __device__ inline void nm_swap32(h8& a, h8& b) {
     b = __builtin_bit_cast(h8, y);
 }
 
+// The power of two 2^e that layer 1's widened codes take from its scale s: e = ceil(log2 s), between -7, down to which
+// the codes keep their bits as halves, and 15.  Codes span the same range whatever their scale; without it hidden values
+// would be as large as those of weights up to 1.75, and leave the halves' range for latents of a few thousand; with it they
+// are at most twice their true size, or below 28 x 65,504 / 128.  (On the accumulator the scale is 32 products a wave and its
+// pixels: k_nm_eval with FP8 weights 452 us instead of 430 for 32 materials of 1024^2 texels, k_shade_ms 528 instead of 506
+// for four cameras with 4 samples.)
+__device__ inline uint32_t nm_first_scale(float s) {
+    int e;
+    if (frexpf(s, &e) == 0.5f) --e;
+    e = max(-7, min(15, e));
+    return __builtin_bit_cast(uint32_t, h2{_Float16(ldexpf(1.f, e)), _Float16(ldexpf(1.f, -e))});
+}
+
 // MLP of the 64 pixels of a wave, one pixel per lane (features f from nm_features); every lane of
 // the wave must call it with the wave fully active.  Returns this lane's 7 clamped outputs.
 //
@@ -188,9 +201,10 @@ __device__ inline void nm_swap32(h8& a, h8& b) {
 // hi / lo pair (nm_split8).
 __device__ inline void nm_mlp_wave(const NmWeights* __restrict__ W, const float f[kNmFeat], float out[kNmOut]) {
     const uint32_t lane = nm_lane();
+    const h2 first = __builtin_bit_cast(h2, W->first);
     h8 a1, a2[2];
     if (W->fp8) {  // uniform: one weight form per decoder
-        a1 = nm_widen_e4m3(W->q1[lane]);
+        a1 = nm_widen_e4m3(W->q1[lane]) * first[0];
         a2[0] = nm_widen_e4m3(W->q2[0][lane]);
         a2[1] = nm_widen_e4m3(W->q2[1][lane]);
     } else {
@@ -211,20 +225,14 @@ __device__ inline void nm_mlp_wave(const NmWeights* __restrict__ W, const float 
     h8 q1h = __builtin_bit_cast(h8, ph), q1l = __builtin_bit_cast(h8, pl);
     nm_swap32(q0h, q1h);  // q0: tile 0's operand (lower lanes the first half, upper lanes the second), q1: tile 1's
     nm_swap32(q0l, q1l);
-    // layer 1's scale goes on its accumulator (1 in the FP16 form): stored codes are up to 1.75 whatever the weights,
-    // and times features of a few thousand they would leave the halves' range (k_nm_eval with FP8 weights, 32 materials of
-    // 1024^2 texels: 452 us, 430 with both scales on the outputs; frames the same)
-    const bool scaled = W->fp8 != 0u;
-    const float s1 = W->scale[0], s2 = W->scale[1];
+    // what is left of both layers' scales goes on the outputs: relu(s x) = s relu(x) for s > 0
+    const float s12 = W->scale[0] * W->scale[1] * float(first[1]);
     uint32_t res[2][4];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         f32x16 acc = {};
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, t == 0 ? q0h : q1h, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, t == 0 ? q0l : q1l, acc, 0, 0, 0);
-        if (scaled)  // uniform
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[r] *= s1;
         f32x16 acc2 = {};
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -248,7 +256,7 @@ __device__ inline void nm_mlp_wave(const NmWeights* __restrict__ W, const float 
         if (r < 3) out[4 + r] = __uint_as_float(res[1][r]);
     }
 #pragma unroll
-    for (int c = 0; c < kNmOut; ++c) out[c] = __builtin_amdgcn_fmed3f(fmaf(out[c], s2, W->b2[c]), 0.f, 1.f);
+    for (int c = 0; c < kNmOut; ++c) out[c] = __builtin_amdgcn_fmed3f(fmaf(out[c], s12, W->b2[c]), 0.f, 1.f);
 }
 
 }  // namespace rsy

@@ -742,7 +742,8 @@ __device__ inline void nm_row(uint4 a, uint4 b, float t, float (&out)[kNmCh]) {
 // kNmEvalW x kNmEvalH texels: lane = column, a wave walks kNmEvalH / 4 rows.
 //
 // kTexel: the slot's three maps share one extent, so that the plain sampler at a texel centre is the
-// texel itself (bilinear weights 1, 0, 0, 0): three loads and seven table reads, against twelve loads
+// texel itself (bilinear weights 1, 0, 0, 0: in FP32 exactly so for extents that are powers of two, for others within
+// the rounding of the coordinates, which reading the texel leaves out): three loads and seven table reads, against twelve loads
 // with addressing and format branches.  Slots whose maps differ in size sample bilinearly
 // (kTexel = false); each launch passes over the other kind's slots.
 //
@@ -916,7 +917,7 @@ __device__ void export_weights(const float* p, NmWeights* W, uint32_t fp8) {
     if (l < 2) W->scale[l] = fp8 ? scale[l] * 256.f : 1.f;
     if (l == 0) {
         W->fp8 = fp8 ? 1u : 0u;
-        W->pad = 0u;
+        W->first = fp8 ? nm_first_scale(scale[0] * 256.f) : 0x3c003c00u;  // 1 and 1
     }
 }
 

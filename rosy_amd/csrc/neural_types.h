@@ -22,7 +22,7 @@ constexpr int kNmStepTables = 19;
 
 // Bytes of the MFMA-operand form of the MLP: the FP16 A operands of both layers (3 x 64 entries of
 // 16 bytes), the same as E4M3 codes (3 x 64 entries of 8 bytes), FP32 b2, two FP32 layer scales,
-// the weight-form flag and padding.
+// the weight-form flag and layer 1's power of two.
 constexpr size_t kNmWeightsBytes = 3 * 64 * 16 + 3 * 64 * 8 + 8 * 4 + 2 * 4 + 2 * 4;
 
 // One decoded material: the material index and its three source maps (texture table indices).
