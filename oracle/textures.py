@@ -1,5 +1,5 @@
 """CPU restatement of the texture pipeline's mip chains -- test infrastructure: the oracle the
-library's mip builder (launch_build_mip, rosy_amd/csrc/bc7.hip) is checked against; nothing in the
+library's mip builder (launch_build_mips, rosy_amd/csrc/bc7.hip) is checked against; nothing in the
 product imports it.
 
 The reference's packager builds each image's chain with NVTT (Packager.cpp:216-308): for sRGB

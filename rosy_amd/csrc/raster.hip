@@ -348,8 +348,8 @@ __device__ inline BlockEntry load_entry(const BlockEntry* blocks, uint32_t b) {
 
 // Stores of a setup block's records and cleared words.  kStream (frames of many blocks, whose records outgrow the caches
 // before anything reads them) writes them past the caches, which stay with the indices and vertices that blocks
-// share: k_setup<2> 83 -> 76 us, the scatter after it 14.5 -> 13.1 and the raster 54 -> 53 at 1M triangles in five
-// views; 269 -> 261, 44.6 -> 37.2 and 102 -> 100 at 2M in eight.  A small frame's raster reads its records from the
+// share: k_setup<2> 82 -> 75 us, the scatter after it 14.1 -> 13.0 and the raster 50.7 -> 49.8 at 1M triangles in five
+// views; 264 -> 259, 44.4 -> 36.9 and 93.2 -> 89.9 at 2M in eight.  A small frame's raster reads its records from the
 // caches: with streamed stores k_setup<1> takes 19.9 instead of 18.9 us and the raster 30.8 instead of 29.7.
 template <bool kStream>
 __device__ inline void store16(void* p, uint4 v) {
@@ -582,8 +582,10 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(const ViewGPU* views, con
     const ViewGPU V = views[view];
     uint32_t* ctr = counters + view * kCtrPerView;
     const uint32_t n = min(ctr[kCtrClip], V.clip_cap);
-    // the output of a view whose setup blocks are too few to clear it (a fill launch a view before: with little to
-    // draw, a frame's time is its launches, 72 and 65.5 us at 640 x 360)
+    // the output of a view whose setup blocks are too few to clear it.  With little to draw, a frame's time is its
+    // launches: 72 us at 640 x 360 with a fill launch a view, 65.5 this way.  Large outputs go at the rate of a fill here,
+    // too (fill and clipper, and the clipper that clears): 66 MB of a 3840 x 2160 view 15.0 and 11.6 us, its 265 MB with
+    // 4 samples 38.1 and 34.5, two views of 66 and 4 MB 21.9 and 13.4.
     if (!V.blend && !V.setup_clear) {
         const uint64_t words = uint64_t(V.width) * V.height * (V.is_shadow ? 1u : 2u * V.samples);
         struct __attribute__((packed, aligned(4))) Four {  // (a caller's buffer may lie at any word)

@@ -620,7 +620,7 @@ __device__ __forceinline__ Fragment shade_pixel(const ShadeLaunch& L, const Shad
 }
 
 // The shaded colour, written once and past the caches (as a pixel's visibility word is read), which stay with vertices,
-// texels and shadow map: k_shade 35.3 -> 34.3 us at 1920 x 1080, 76.8 -> 72.4 at 2560 x 1440.
+// texels and shadow map: k_shade 35.3 -> 34.1 us at 1920 x 1080, 73.4 -> 69.5 at 2560 x 1440.
 typedef float f32x4_store __attribute__((ext_vector_type(4)));
 __device__ inline void store_color(const ShadeView& V, size_t o, float4 c) {
     const f32x4_store v = {c.x, c.y, c.z, c.w};
