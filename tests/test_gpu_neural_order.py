@@ -67,3 +67,37 @@ def test_run_repeats(region, batch):
             scene.close()
     for a, b in zip(*runs):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("n,spread", [(31, 0.0), (33, 0.0), (300, 0.0), (520, 0.1)])
+def test_crowded_cells(n, spread):
+    """The same sum where one cell has few samples, more than a wave takes one by one, and several chunks of them."""
+    rng = np.random.default_rng(n)
+    scene, r = renderer()
+    try:
+        latent = 8
+        r.neural_init(latent_size=latent, region=8, seed=5)
+        r.neural_set_params(rng.uniform(-0.8, 0.8, (2, latent, latent, 8)).astype(np.float32),
+                            rng.uniform(-0.5, 0.5, 583).astype(np.float32))
+        uv = (0.4 + (spread + 0.02) * rng.random((n, 2))).astype(np.float32)
+        target = rng.random((n, 7)).astype(np.float32)
+
+        def gradient(rows):
+            others = np.setdiff1d(np.arange(n), rows)
+            order = np.concatenate([rows, others])
+            material = np.r_[np.zeros(len(rows), np.uint32), np.ones(len(others), np.uint32)]
+            return r.neural_gradients(material, uv[order], target[order])[2][0]
+
+        alone = [gradient(np.array([i])) for i in range(n)]
+        base = np.floor(uv * np.float32(latent) - np.float32(0.5)).astype(int)
+        want = np.zeros_like(alone[0])
+        for chunk in range(0, n, 256):  # the kernel takes 256 samples at a time
+            for dy, dx in ((0, 0), (0, 1), (1, 0), (1, 1)):
+                for i in range(chunk, min(chunk + 256, n)):
+                    x, y = (base[i] + (dx, dy)) % latent
+                    want[y, x] += alone[i][y, x]
+        got = gradient(np.arange(n))
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.abs(got - want).max()
+    finally:
+        r.close()
+        scene.close()
